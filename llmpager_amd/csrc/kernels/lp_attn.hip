@@ -186,130 +186,268 @@ extern "C" __global__ void __launch_bounds__(256) lp_strided_copy(const StridedC
 // ---------------------------------------------------------------------------
 // Decode attention, one query per head, split over positions (attn_decode_f32
 // / _f16kv, decode.cu:172-325; mla_attn_decode_f32, mla.cu:51-111).  Grid
-// (heads, splits), 256 threads.  Split s of head h takes positions
-// [s span, min((s + 1) span, seq_len)): each thread scores whole positions
-// (its key row against the query staged in LDS), the workgroup takes their
-// max and the sum of exp(score - max), then each thread accumulates output
-// dimensions over the split's positions.  One split writes out[h] = acc / sum;
-// more write partial records {max, sum, acc[out_dim]} that lp_attn_combine
-// merges (an empty split records {-inf, 0, 0...}).
+// (kv heads x blocks of kAttnHeads query heads of one kv head, splits), 256
+// threads.
+//
+// One token's attention is a chain of memory round trips, not bytes (3 MB at
+// 1,500 positions of 4 kv heads), so a workgroup brings a chunk of rows'
+// keys and values in by one burst of coalesced loads, fp32 in LDS, and all
+// query heads of the kv head use them: each row is read once for the group.
+//   scores   thread (rows t % 32 and t % 32 + 32, head t / 32): fused
+//            multiply-adds over the row, the rows padded by 16 bytes so 16 lanes' 16-byte reads
+//            cover the banks;
+//   softmax  online over the chunks, each head's scores in half a wave;
+//   context  thread (4 columns, kAttnHeads / slots heads): rows from LDS,
+//            probabilities broadcast.
+// One split writes out[h] = acc / sum; more write records {max, sum,
+// acc[out_dim]} that lp_attn_combine merges.  (One thread per key row and a
+// workgroup per query head before: 38.4 us at 32 heads on 4 kv heads, 1,502
+// f16 rows of 128; 11.3 now.  The merge 16.1 before, 4.5 now.)
 // ---------------------------------------------------------------------------
 namespace {
 
+// Rows [0, rows) of a cache at element `at` as fp32 in LDS, row stride rs
+// floats, columns past n zero.  A vector piece is 16 bytes; four pieces per
+// thread are loaded before the first is stored.
 template <bool F16>
-__device__ __forceinline__ float cache_at(uint64_t base, size_t i) {
-    if constexpr (F16)
-        return half_bits_to_f32(dptr<const uint16_t>(base)[i]);
-    else
-        return dptr<const float>(base)[i];
-}
-
-// dot(q, row) over n elements of an f32 or f16 cache row; vector loads when
-// the row and n allow them
-template <bool F16>
-__device__ __forceinline__ float row_dot(const float* qs, uint64_t base, size_t row0, int n) {
-    float dot = 0.0f;
-    if constexpr (F16) {
-        if ((n & 7) == 0 && ((base + row0 * 2) & 15) == 0) {
-            const uint4* r = reinterpret_cast<const uint4*>(base + row0 * 2);
-            for (int c = 0; c < (n >> 3); ++c) {
-                const uint4 u = r[c];
-                const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
+struct AttnStage {
+    static constexpr int kPer = F16 ? 8 : 4;
+    uint64_t src;  // address of the first row
+    float* dst;
+    int row_bytes, rs, n, n4, rows, pieces;
+    bool vec;
+    uint4 u[4];
+    __device__ __forceinline__ AttnStage(float* d, int rs_, uint64_t base, size_t at, int row_stride, int rows_, int n_,
+                                         int n4_)
+        : src(base + at * (F16 ? 2 : 4)), dst(d), row_bytes(row_stride * (F16 ? 2 : 4)), rs(rs_), n(n_), n4(n4_),
+          rows(rows_) {
+        vec = (n & (kPer - 1)) == 0 && (src & 15) == 0 && (row_bytes & 15) == 0;
+        pieces = vec ? rows * (n / kPer) : 0;
+    }
+    __device__ __forceinline__ void load(int i0) {
+        const int per = n / kPer;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    dot = __builtin_fmaf(qs[8 * c + 2 * j], half_bits_to_f32(wv[j]), dot);
-                    dot = __builtin_fmaf(qs[8 * c + 2 * j + 1], half_bits_to_f32(wv[j] >> 16), dot);
+        for (int j = 0; j < 4; ++j) {
+            const int i = min(i0 + 256 * j + (int)threadIdx.x, pieces - 1), r = i / per;
+            u[j] = *gptr<uint4>(src + (uint64_t)((uint32_t)r * (uint32_t)row_bytes + 16u * (uint32_t)(i - r * per)));
+        }
+    }
+    __device__ __forceinline__ void store(int i0) {
+        const int per = n / kPer;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + 256 * j + (int)threadIdx.x, r = i / per;
+            if (i >= pieces) break;
+            float* o = dst + r * rs + (i - r * per) * kPer;
+            if constexpr (F16) {
+                reinterpret_cast<float4*>(o)[0] =
+                    make_float4(half_bits_to_f32(u[j].x), half_bits_to_f32(u[j].x >> 16), half_bits_to_f32(u[j].y),
+                                half_bits_to_f32(u[j].y >> 16));
+                reinterpret_cast<float4*>(o)[1] =
+                    make_float4(half_bits_to_f32(u[j].z), half_bits_to_f32(u[j].z >> 16), half_bits_to_f32(u[j].w),
+                                half_bits_to_f32(u[j].w >> 16));
+            } else {
+                *reinterpret_cast<uint4*>(o) = u[j];
+            }
+        }
+    }
+    __device__ __forceinline__ void scalar() {  // widths or addresses that do not make 16-byte pieces
+        for (int i = threadIdx.x; i < rows * 4 * n4; i += 256) {
+            const int r = i / (4 * n4), c = i - r * 4 * n4;
+            const uint64_t row = src + (uint64_t)r * (uint32_t)row_bytes;
+            float v = 0.0f;
+            if (c < n) {
+                if constexpr (F16)
+                    v = half_bits_to_f32(gptr<uint16_t>(row)[c]);
+                else
+                    v = gptr<float>(row)[c];
+            }
+            dst[r * rs + c] = v;
+        }
+    }
+};
+
+// HPT: query heads per thread in the context pass (1 up to 128 columns, 2 up
+// to 256, 4 up to 512, 8 up to 1024).
+template <bool F16, int HPT>
+__device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, sp = blockIdx.y;
+    const int blocks = (a.group + kAttnHeads - 1) / kAttnHeads;
+    const int kvh = blockIdx.x / blocks, h0 = kvh * a.group + (blockIdx.x - kvh * blocks) * kAttnHeads;
+    const int nh = min(kAttnHeads, (kvh + 1) * a.group - h0);
+    const int d4 = (a.dot_dim + 3) >> 2, o4 = (a.out_dim + 3) >> 2;
+    const int krs = attn_row_floats(a.dot_dim), vrs = a.shared_kv ? krs : attn_row_floats(a.out_dim);
+    float* qs = reinterpret_cast<float*>(lds);  // [kAttnHeads][4 d4]
+    float* pr = qs + kAttnHeads * 4 * d4;       // [kAttnHeads][32]
+    float* al = pr + kAttnHeads * kAttnRows;    // [kAttnHeads]: the chunk's rescaling
+    float* kt = al + kAttnHeads;                // [rows][krs]
+    float* vt = a.shared_kv ? kt : kt + a.rows * krs;
+    const float* q = dptr<const float>(a.q) + (size_t)h0 * a.dot_dim;
+    for (int i = tid; i < kAttnHeads * 4 * d4; i += 256) {
+        const int h = i / (4 * d4), d = i - h * 4 * d4;
+        qs[i] = h < nh && d < a.dot_dim ? q[(size_t)h * a.dot_dim + d] : 0.0f;
+    }
+    const size_t kv_off = (size_t)kvh * a.kv_stride;
+    const int p0 = sp * a.span, p1 = min(a.seq_len, p0 + a.span);
+    const int pl = tid & 31, hl = tid >> 5;  // score pass: row, head
+    float m = -INFINITY, l = 0.0f;           // head hl's running max and sum (in its 32 lanes alike)
+    // context pass: columns 4 c .. 4 c + 3, heads hs, hs + slots, ...
+    const int quads = o4 <= 32 ? 32 : o4 <= 64 ? 64 : o4 <= 128 ? 128 : 256;
+    const int c = tid & (quads - 1), hs = tid / quads, slots = 256 / quads;
+    float4 acc[HPT];
+#pragma unroll
+    for (int j = 0; j < HPT; ++j) acc[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int p = p0; p < p1; p += a.rows) {
+        const int n = min(a.rows, p1 - p);
+        if (p > p0) __syncthreads();  // the previous chunk's rows are read
+        const size_t at = kv_off + (size_t)p * a.row_stride;
+        AttnStage<F16> K(kt, krs, a.k, at, a.row_stride, n, a.dot_dim, d4);
+        AttnStage<F16> V(vt, vrs, a.v, at, a.row_stride, a.shared_kv ? 0 : n, a.out_dim, o4);
+        for (int i = 0; i < max(K.pieces, V.pieces); i += 1024) {  // keys and values in one burst
+            if (i < K.pieces) K.load(i);
+            if (i < V.pieces) V.load(i);
+            if (i < K.pieces) K.store(i);
+            if (i < V.pieces) V.store(i);
+        }
+        if (!K.vec) K.scalar();
+        if (!V.vec) V.scalar();
+        __syncthreads();
+        // rows pl and pl + 32 together: one read of q for two
+        float s0 = -INFINITY, s1 = -INFINITY;
+        if (pl < n) {
+            const float4* kr0 = reinterpret_cast<const float4*>(kt + pl * krs);
+            const float4* kr1 = reinterpret_cast<const float4*>(kt + min(pl + 32, n - 1) * krs);
+            const float4* qr = reinterpret_cast<const float4*>(qs + hl * 4 * d4);
+            s0 = s1 = 0.0f;
+#pragma unroll 8
+            for (int i = 0; i < d4; ++i) {
+                const float4 x0 = kr0[i], x1 = kr1[i], y = qr[i];
+                s0 = __builtin_fmaf(y.x, x0.x, s0);
+                s1 = __builtin_fmaf(y.x, x1.x, s1);
+                s0 = __builtin_fmaf(y.y, x0.y, s0);
+                s1 = __builtin_fmaf(y.y, x1.y, s1);
+                s0 = __builtin_fmaf(y.z, x0.z, s0);
+                s1 = __builtin_fmaf(y.z, x1.z, s1);
+                s0 = __builtin_fmaf(y.w, x0.w, s0);
+                s1 = __builtin_fmaf(y.w, x1.w, s1);
+            }
+            s0 *= a.scale;
+            s1 = pl + 32 < n ? s1 * a.scale : -INFINITY;
+        }
+        float mx = fmaxf(s0, s1);
+#pragma unroll
+        for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, shfl_xor(mx, o));
+        const float mn = fmaxf(m, mx);
+        // every score so far -inf: nothing to rescale, nothing added
+        const float alpha = mn == -INFINITY ? 1.0f : expf(m - mn);
+        const float e0 = mn == -INFINITY ? 0.0f : expf(s0 - mn);
+        const float e1 = mn == -INFINITY ? 0.0f : expf(s1 - mn);
+        float sum = e0 + e1;
+#pragma unroll
+        for (int o = 16; o >= 1; o >>= 1) sum += shfl_xor(sum, o);
+        l = __builtin_fmaf(l, alpha, sum);
+        m = mn;
+        pr[hl * kAttnRows + pl] = e0;
+        pr[hl * kAttnRows + pl + 32] = e1;
+        if (pl == 0) al[hl] = alpha;
+        __syncthreads();
+        if (c < o4) {
+#pragma unroll
+            for (int j = 0; j < HPT; ++j) {
+                const float f = al[(hs + j * slots) & (kAttnHeads - 1)];
+                acc[j] = make_float4(acc[j].x * f, acc[j].y * f, acc[j].z * f, acc[j].w * f);
+            }
+#pragma unroll 8
+            for (int r = 0; r < n; ++r) {
+                const float4 v = *reinterpret_cast<const float4*>(vt + r * vrs + 4 * c);
+#pragma unroll
+                for (int j = 0; j < HPT; ++j) {
+                    const float w = pr[((hs + j * slots) & (kAttnHeads - 1)) * kAttnRows + r];
+                    acc[j].x = __builtin_fmaf(w, v.x, acc[j].x);
+                    acc[j].y = __builtin_fmaf(w, v.y, acc[j].y);
+                    acc[j].z = __builtin_fmaf(w, v.z, acc[j].z);
+                    acc[j].w = __builtin_fmaf(w, v.w, acc[j].w);
                 }
             }
-            return dot;
-        }
-    } else {
-        if ((n & 3) == 0 && ((base + row0 * 4) & 15) == 0) {
-            const float4* r = reinterpret_cast<const float4*>(base + row0 * 4);
-            for (int c = 0; c < (n >> 2); ++c) {
-                const float4 u = r[c];
-                dot = __builtin_fmaf(qs[4 * c], u.x, dot);
-                dot = __builtin_fmaf(qs[4 * c + 1], u.y, dot);
-                dot = __builtin_fmaf(qs[4 * c + 2], u.z, dot);
-                dot = __builtin_fmaf(qs[4 * c + 3], u.w, dot);
-            }
-            return dot;
         }
     }
-    for (int d = 0; d < n; ++d) dot = __builtin_fmaf(qs[d], cache_at<F16>(base, row0 + d), dot);
-    return dot;
+    // each head's max and sum to the threads that hold its columns
+    __syncthreads();
+    if (pl == 0) pr[2 * hl] = m, pr[2 * hl + 1] = l;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < HPT; ++j) {
+        const int h = hs + j * slots;
+        if (h >= nh || c >= o4) continue;
+        const float f = a.splits == 1 ? 1.0f / pr[2 * h + 1] : 1.0f;
+        float* o = a.splits == 1 ? dptr<float>(a.out) + (size_t)(h0 + h) * a.out_dim
+                                 : dptr<float>(a.scratch) + (size_t)(h0 + h) * a.scratch_stride +
+                                       (size_t)sp * (a.out_dim + 2) + 2;
+        const float v[4] = {acc[j].x * f, acc[j].y * f, acc[j].z * f, acc[j].w * f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (4 * c + i < a.out_dim) o[4 * c + i] = v[i];
+        if (a.splits > 1 && c == 0) {
+            o[-2] = pr[2 * h];
+            o[-1] = pr[2 * h + 1];
+        }
+    }
 }
 
-constexpr int kAttnMaxDot = 1024;
-
 template <bool F16>
-__device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
-    __shared__ float qs[kAttnMaxDot];
-    __shared__ float sc[kAttnSpanMax];
-    __shared__ float red[4];
-    const int h = blockIdx.x, sp = blockIdx.y, tid = threadIdx.x;
-    const uint64_t kv_off = (uint64_t)(h / a.group) * a.kv_stride;
-    const float* q = dptr<const float>(a.q) + (size_t)h * a.dot_dim;
-    for (int d = tid; d < a.dot_dim; d += 256) qs[d] = q[d];
-    __syncthreads();
-    const int p0 = sp * a.span;
-    const int p1 = min(a.seq_len, p0 + a.span);
-    float lmax = -INFINITY;
-    for (int p = p0 + tid; p < p1; p += 256) {
-        const float s = row_dot<F16>(qs, a.k, kv_off + (size_t)p * a.row_stride, a.dot_dim) * a.scale;
-        sc[p - p0] = s;
-        lmax = fmaxf(lmax, s);
-    }
-    const float m = block_max(lmax, red);
-    float lsum = 0.0f;
-    for (int p = p0 + tid; p < p1; p += 256) {
-        const float e = expf(sc[p - p0] - m);
-        sc[p - p0] = e;
-        lsum += e;
-    }
-    const float l = block_sum(lsum, red);
-    float* part = dptr<float>(a.scratch) + (size_t)h * a.scratch_stride + (size_t)sp * (a.out_dim + 2);
-    for (int d = tid; d < a.out_dim; d += 256) {
-        float acc = 0.0f;
-        for (int p = p0; p < p1; ++p)
-            acc = __builtin_fmaf(sc[p - p0], cache_at<F16>(a.v, kv_off + (size_t)p * a.row_stride + d), acc);
-        if (a.splits == 1)
-            dptr<float>(a.out)[(size_t)h * a.out_dim + d] = acc * (1.0f / l);
-        else
-            part[2 + d] = acc;
-    }
-    if (a.splits > 1 && tid == 0) {
-        part[0] = m;
-        part[1] = l;
-    }
+__device__ __forceinline__ void attn_split(const AttnArgs& a) {
+    const int o4 = (a.out_dim + 3) >> 2;
+    if (o4 <= 32)
+        attn_split_body<F16, 1>(a);
+    else if (o4 <= 64)
+        attn_split_body<F16, 2>(a);
+    else if (o4 <= 128)
+        attn_split_body<F16, 4>(a);
+    else
+        attn_split_body<F16, 8>(a);
 }
 
 }  // namespace
 
-extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f32(const AttnArgs a) { attn_split_body<false>(a); }
-extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f16(const AttnArgs a) { attn_split_body<true>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f32(const AttnArgs a) { attn_split<false>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f16(const AttnArgs a) { attn_split<true>(a); }
 
 // Merge of the split records: out[h][d] = sum_s e^(m_s - M) acc_s[d] /
-// sum_s e^(m_s - M) l_s, M = max_s m_s.  Grid heads, 256 threads.
+// sum_s e^(m_s - M) l_s, M = max_s m_s.  Grid (heads, ceil(out_dim / 64)),
+// 256 threads: the weights to LDS, one split per thread, then thread (column
+// d, group g) sums the splits g, g + 4, ... and the groups meet in LDS, so
+// that the records come in a few bursts instead of one dependent load per
+// split.
 extern "C" __global__ void __launch_bounds__(256) lp_attn_combine(const AttnArgs a) {
-    const int h = blockIdx.x;
+    __shared__ float wsh[kAttnMaxSplits];
+    __shared__ float red[4];
+    __shared__ float part[4][64];
+    const int h = blockIdx.x, tid = threadIdx.x;
     const float* base = dptr<const float>(a.scratch) + (size_t)h * a.scratch_stride;
     const int rec = a.out_dim + 2;
-    float M = -INFINITY;
-    for (int s = 0; s < a.splits; ++s) M = fmaxf(M, base[(size_t)s * rec]);
-    float den = 0.0f;
-    for (int s = 0; s < a.splits; ++s) {
-        const float ms = base[(size_t)s * rec];
-        if (ms != -INFINITY) den = __builtin_fmaf(expf(ms - M), base[(size_t)s * rec + 1], den);
-    }
-    for (int d = threadIdx.x; d < a.out_dim; d += 256) {
-        float num = 0.0f;
-        for (int s = 0; s < a.splits; ++s) {
-            const float ms = base[(size_t)s * rec];
-            if (ms != -INFINITY) num = __builtin_fmaf(expf(ms - M), base[(size_t)s * rec + 2 + d], num);
+    const float ms = tid < a.splits ? base[(size_t)tid * rec] : -INFINITY;
+    const float ls = tid < a.splits ? base[(size_t)tid * rec + 1] : 0.0f;
+    const float M = block_max(ms, red);
+    const float w = ms == -INFINITY ? 0.0f : expf(ms - M);
+    const float den = block_sum(w * ls, red);
+    if (tid < a.splits) wsh[tid] = ms == -INFINITY ? -1.0f : w;  // -1: an empty split
+    __syncthreads();
+    const int d = blockIdx.y * 64 + (tid & 63), g = tid >> 6;
+    float num = 0.0f;
+    if (d < a.out_dim) {
+        const float* col = base + 2 + d;
+#pragma unroll 8
+        for (int s = g; s < a.splits; s += 4) {
+            const float v = col[(size_t)s * rec], ws = wsh[s];
+            num = ws < 0.0f ? num : __builtin_fmaf(ws, v, num);
         }
-        dptr<float>(a.out)[(size_t)h * a.out_dim + d] = num / den;
     }
+    part[g][tid & 63] = num;
+    __syncthreads();
+    if (g == 0 && d < a.out_dim)
+        dptr<float>(a.out)[(size_t)h * a.out_dim + d] =
+            ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) / den;
 }
 
 // ---------------------------------------------------------------------------

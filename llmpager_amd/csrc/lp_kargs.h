@@ -236,8 +236,20 @@ struct StridedCopyArgs {            // kernels.rs:386-404 (strided_copy_f32)
 // {max, sum, acc[out_dim]} at scratch + h * scratch_stride + s * (out_dim + 2)
 // that lp_attn_combine merges.  Keys of head h: k + (h / group) * kv_stride,
 // row p at p * row_stride elements, `dot_dim` wide; values likewise from v,
-// `out_dim` wide.  GQA decode has k != v; MLA reads both from its one cache.
-constexpr int kAttnSpanMax = 1024;  // positions per split (LDS scores)
+// `out_dim` wide.  GQA decode has k != v; MLA reads both from its one cache
+// (shared_kv).  A workgroup takes kAttnHeads query heads of one kv head and
+// walks its span in chunks of `rows` (kAttnRows, fewer where the LDS asks).
+constexpr int kAttnSpanMax = 1024;   // more positions than this per record are refused
+constexpr int kAttnHeads = 8;
+constexpr int kAttnRows = 64;
+constexpr int kAttnMaxSplits = 256;  // lp_attn_combine: one split per thread
+// LDS: q [kAttnHeads] rows, probabilities, rescalings, then the chunk's rows,
+// 16 bytes of pad each.
+LPK_HD constexpr int attn_row_floats(int n) { return ((n + 3) & ~3) + 4; }
+LPK_HD constexpr int attn_lds_bytes(int dot_dim, int out_dim, bool shared_kv, int rows) {
+    return 4 * (kAttnHeads * ((dot_dim + 3) & ~3) + kAttnHeads * kAttnRows + kAttnHeads +
+                rows * (attn_row_floats(dot_dim) + (shared_kv ? 0 : attn_row_floats(out_dim))));
+}
 struct AttnArgs {
     uint64_t q, k, v, out, scratch;
     uint64_t kv_stride;             // elements between kv heads' caches
@@ -246,6 +258,8 @@ struct AttnArgs {
     int32_t splits, span, scratch_stride;
     float scale;
     int32_t f16;                    // caches hold IEEE half (else f32)
+    int32_t rows;                   // rows per chunk (a multiple of 8, at most kAttnRows)
+    int32_t shared_kv;              // values are the first out_dim columns of the key rows
     int32_t pad0;
 };
 

@@ -719,30 +719,32 @@ int lp_strided_copy(lp_ctx* c, uint64_t src, int src_stride, int src_off, uint64
     return launch(c, kStridedCopy, dim3(grid_1d(n_vecs * n)), dim3(256), 0, s, a);
 }
 
-// Split decode attention: splits so that the grid fills the chip, each split
-// at most kAttnSpanMax positions (and at least 32), the partial records in
-// the caller's scratch [heads, max_seq] (splits * (out_dim + 2) floats per
-// head); one split writes the output directly.
+// Split decode attention: a workgroup per (kAttnHeads query heads of one kv
+// head, split), about two per CU and each split whole chunks of rows, the
+// partial records in the caller's scratch [heads, max_seq] (splits * (out_dim
+// + 2) floats per head); one split writes the output directly.
 static int attn_launch(lp_ctx* c, AttnArgs a, int max_seq, lp_stream s) {
     if (a.seq_len < 1 || a.seq_len > max_seq) return fail(LP_E_INVALID, "attention: need 1 <= seq_len <= max_seq");
     if (a.dot_dim < 1 || a.dot_dim > 1024 || a.out_dim < 1 || a.out_dim > a.row_stride || a.dot_dim > a.row_stride)
         return fail(LP_E_UNSUPPORTED, "attention: dims must be 1..1024 and fit a cache row");
     const int by_span = (a.seq_len + kAttnSpanMax - 1) / kAttnSpanMax;
     const int by_scratch = max_seq / (a.out_dim + 2);
-    int splits = std::max(1, (2 * c->cus + a.heads - 1) / a.heads);
-    splits = std::min(splits, std::max(1, (a.seq_len + 31) / 32));
-    splits = std::min(splits, std::max(1, by_scratch));
-    splits = std::max(splits, by_span);
-    if (splits > 1 && splits > by_scratch)
+    if (by_span > 1 && by_span > by_scratch)
         return fail(LP_E_UNSUPPORTED, "attention: the scratch cannot hold the split records");
+    a.rows = kAttnRows;
+    while (a.rows > 8 && (size_t)attn_lds_bytes(a.dot_dim, a.out_dim, a.shared_kv, a.rows) > c->max_lds) a.rows >>= 1;
+    const int wgs = a.heads / a.group * ((a.group + kAttnHeads - 1) / kAttnHeads);
+    int splits = std::max(1, (2 * c->cus + wgs - 1) / wgs);
+    splits = std::min({splits, (a.seq_len + a.rows - 1) / a.rows, std::max(1, by_scratch), kAttnMaxSplits});
     a.span = (a.seq_len + splits - 1) / splits;
+    a.span = (a.span + a.rows - 1) / a.rows * a.rows;
     a.splits = (a.seq_len + a.span - 1) / a.span;
     a.scratch_stride = max_seq;
-    if (int r = launch(c, a.f16 ? kAttnSplitF16 : kAttnSplitF32, dim3((unsigned)a.heads, (unsigned)a.splits),
-                       dim3(256), 0, s, a))
+    if (int r = launch(c, a.f16 ? kAttnSplitF16 : kAttnSplitF32, dim3((unsigned)wgs, (unsigned)a.splits), dim3(256),
+                       (size_t)attn_lds_bytes(a.dot_dim, a.out_dim, a.shared_kv, a.rows), s, a))
         return r;
     if (a.splits == 1) return LP_OK;
-    return launch(c, kAttnCombine, dim3((unsigned)a.heads), dim3(256), 0, s, a);
+    return launch(c, kAttnCombine, dim3((unsigned)a.heads, (unsigned)((a.out_dim + 63) / 64)), dim3(256), 0, s, a);
 }
 
 int lp_attn_decode(lp_ctx* c, uint64_t q, uint64_t kcache, uint64_t vcache, uint64_t out, uint64_t scratch,
@@ -777,6 +779,7 @@ int lp_mla_attn_decode(lp_ctx* c, uint64_t q, uint64_t cache, uint64_t ctx, uint
     a.out = ctx;
     a.scratch = scratch;
     a.kv_stride = 0;  // one cache shared by every head (MQA)
+    a.shared_kv = 1;
     a.heads = heads;
     a.group = heads;
     a.dot_dim = qk_dim;

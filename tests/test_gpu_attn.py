@@ -195,3 +195,47 @@ def test_mla_batch_config5(cuda, K, B, qstd):
     # at B = 16 the sequences' lengths vary (full, ragged, one position)
     seqs = [4096] if B == 1 else [4096, 4095, 1, 64, 65, 2048, 3000, 4096, 17, 1000, 4032, 129, 4096, 511, 2, 3333]
     _mla_batch(cuda, K, 16, 576, 512, seqs, 4096, 0.0722, qstd, 100 + B)
+
+
+# The split kernel's edges: query heads per kv head around its blocks of 8
+# (1, 3, 8, 9, 16), row widths that make 16-byte pieces and that do not (f16:
+# 20; f32: 18), wide rows (fewer rows per chunk), lengths around a chunk of 32
+# rows, a scratch that holds one record (one split, many chunks), and a cache
+# address off 16 bytes.  Bound: a score's fp32 chain is off by at most
+# hd 2^-24 scale sum|q k| (|q k| <= 2: 2 sqrt(hd) hd 2^-24 = 1.7e-4 at
+# hd 128), which moves each probability by that relative amount; the outputs
+# are averages of values in [-1, 1].
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("heads,kvh,hd,seq,ms,off", [
+    (2, 2, 128, 31, 40, 0), (6, 2, 128, 32, 1000, 0), (16, 2, 128, 33, 1000, 8), (9, 1, 64, 65, 700, 0),
+    (16, 1, 256, 1025, 2000, 0), (3, 1, 20, 100, 300, 0), (4, 2, 18, 97, 97, 0), (8, 1, 512, 200, 520, 0),
+    (2, 1, 1024, 77, 100, 0), (8, 4, 128, 1000, 131, 0), (32, 4, 128, 4000, 4096, 4)])
+def test_attn_decode_edges(cuda, K, f16, heads, kvh, hd, seq, ms, off):
+    seq = min(seq, ms)
+    rng = np.random.default_rng(hd + seq)
+    scale = 1.0 / np.sqrt(hd)
+    q = _rnd(rng, heads * hd) * 2
+    dt = np.float16 if f16 else np.float32
+    k, v = (_rnd(rng, kvh * ms * hd).astype(dt) for _ in range(2))
+    pad = np.zeros(off // dt().itemsize, dt)
+    dq, dk, dv = cuda.upload(q), cuda.upload(np.concatenate([pad, k])), cuda.upload(np.concatenate([pad, v]))
+    dout, dscr = cuda.alloc_device(heads * hd * 4), cuda.alloc_device(heads * ms * 4)
+    K.attn_decode(dq, dk + off, dv + off, dout, dscr, heads, kvh, hd, seq, ms, scale, f16)
+    bits = np.uint16 if f16 else np.float32
+    want = O.attn_decode(q, k.view(bits), v.view(bits), heads, kvh, hd, seq, ms, scale, f16)
+    tol = 2.0 * np.sqrt(hd) * hd * 2.0 ** -24
+    assert worst_rel(cuda.download(dout, (heads * hd,), np.float32), want) <= max(tol, 2e-5)
+    _free(cuda, dq, dk, dv, dout, dscr)
+
+
+@pytest.mark.parametrize("heads,qk,cd,seq,ms", [(17, 576, 512, 33, 600), (8, 640, 512, 1100, 1100), (1, 30, 18, 40, 64)])
+def test_mla_attn_decode_edges(cuda, K, heads, qk, cd, seq, ms):
+    rng = np.random.default_rng(seq)
+    scale = 1.0 / np.sqrt(qk)
+    q, cache = _rnd(rng, heads * qk) * 2, _rnd(rng, ms * qk)
+    dq, dc = cuda.upload(q), cuda.upload(cache)
+    dctx, dscr = cuda.alloc_device(heads * cd * 4), cuda.alloc_device(heads * ms * 4)
+    K.mla_attn_decode(dq, dc, dctx, dscr, heads, qk, cd, seq, ms, scale)
+    want = O.mla_attn_decode(q, cache[:seq * qk], heads, qk, cd, seq, scale)
+    assert worst_rel(cuda.download(dctx, (heads * cd,), np.float32), want) <= 2.0 * np.sqrt(qk) * qk * 2.0 ** -24
+    _free(cuda, dq, dc, dctx, dscr)
