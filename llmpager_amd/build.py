@@ -3,7 +3,7 @@
 Outputs (under llmpager_amd/lib/):
   lp_basic.hsaco, lp_moe.hsaco,
   lp_gemm.hsaco, lp_attn.hsaco,
-  lp_step.hsaco                   kernels, hipcc --genco --offload-arch=gfx950
+  lp_step.hsaco, lp_mid.hsaco     kernels, hipcc --genco --offload-arch=gfx950
   libllmpager_hip.so              host runtime (g++), loads the code objects
                                   with hipModuleLoad at lp_init
 
@@ -24,7 +24,8 @@ OUT = os.path.join(HERE, "lib")
 ROOT = os.path.dirname(HERE)
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-KERNEL_SOURCES = ["lp_basic.hip", "lp_moe.hip", "lp_gemm.hip", "lp_attn.hip", "lp_step.hip"]
+KERNEL_SOURCES = ["lp_basic.hip", "lp_moe.hip", "lp_gemm.hip", "lp_attn.hip", "lp_step.hip",
+                  "lp_mid.hip"]
 HOST_SOURCES = ["lp_runtime.cpp", "lp_synth.cpp", "lp_cache.cpp", "lp_pager.cpp", "lp_pack.cpp"]
 HOST_HIP_SOURCES = ["lp_noalloc.hip"]
 

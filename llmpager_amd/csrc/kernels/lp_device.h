@@ -399,6 +399,31 @@ __device__ __forceinline__ void write_h16_words(const float* row, int cols, int 
     }
 }
 
+// The same words of the row's hi and lo images: x 2^-e = hi + lo, lo the
+// rounding of what hi leaves (22 significant bits together).
+__device__ __forceinline__ void write_h16_words2(const float* row, int cols, int e, uint8_t* img, uint8_t* img_lo,
+                                                 int first, int step) {
+    const int ng = cols >> 5, nw = 4 * lpk::frag_ngp(cols);
+    for (int w = first; w < nw; w += step) {
+        const int g = w >> 2, j = w & 3;
+        float v[8], r[8];
+        float4 f0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), f1 = f0;
+        if (g < ng) {
+            f0 = *reinterpret_cast<const float4*>(row + g * 32 + j * 8);
+            f1 = *reinterpret_cast<const float4*>(row + g * 32 + j * 8 + 4);
+        }
+        v[0] = f0.x; v[1] = f0.y; v[2] = f0.z; v[3] = f0.w;
+        v[4] = f1.x; v[5] = f1.y; v[6] = f1.z; v[7] = f1.w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float s = __builtin_ldexpf(v[i], -e);
+            r[i] = s - (float)(_Float16)s;  // exact
+        }
+        reinterpret_cast<uint4*>(img)[w] = h16_word(v, e);
+        reinterpret_cast<uint4*>(img_lo)[w] = h16_word(r, 0);
+    }
+}
+
 // The fp16 image of an fp32 row (global memory or LDS) and its exponent
 // (*exp_out), by the whole workgroup (every thread calls it).
 __device__ __forceinline__ void write_h16_image(const float* row, int cols, uint8_t* img, int* exp_out) {

@@ -357,7 +357,11 @@ extern "C" __global__ void __launch_bounds__(256) lp_moe_ximage(const RouteArgs 
     }
     if (a.make_xf & kImgF16) {
         const int e = h16_exp(row_absmax_wave(row, H, lane, 64));
-        write_h16_words(row, H, e, dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(H), lane, 64);
+        uint8_t* img = dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(H);
+        if (a.make_xf & kImgF16Lo)
+            write_h16_words2(row, H, e, img, img + (size_t)a.T * himage_bytes(H), lane, 64);
+        else
+            write_h16_words(row, H, e, img, lane, 64);
         if (lane == 0) dptr<int>(a.W.xexp)[t] = e;
     }
 }
@@ -893,6 +897,17 @@ extern "C" __global__ void __launch_bounds__(1024) lp_moe_disp_scan(const RouteA
     int total, nu;
     const int g0 = block_excl_scan(tot, scan_sh, &total);
     const int u = block_excl_scan(tot > 0 ? 1 : 0, scan_sh, &nu);
+    // the tile list of the kernels that take a large batch's experts in
+    // blocks of tile_tokens tokens: (entry << 16) | block, by entry
+    if (a.tile_tokens > 0) {
+        const int blocks = (tot + a.tile_tokens - 1) / a.tile_tokens;
+        int ntiles;
+        const int t0 = block_excl_scan(blocks, scan_sh, &ntiles);
+        int* tiles = dptr<int>(a.tiles);
+        for (int b = 0; b < blocks; ++b)
+            if (t0 + b < a.max_tiles) tiles[t0 + b] = (u << 16) | b;
+        if (tid == 0) dptr<int>(a.W.meta)[2] = min(ntiles, a.max_tiles);
+    }
     ExpertEntry* et = dptr<ExpertEntry>(a.W.et);
     if (tid < E) {
         dptr<int>(a.W.gs)[tid] = g0;

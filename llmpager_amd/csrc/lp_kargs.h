@@ -348,7 +348,7 @@ struct Workspace {
     uint64_t sh_perm;    // shared MLP: i32 [T], t
     uint64_t sh_act;     // shared MLP: f32 [T, shared_inter]
     uint64_t sh_y;       // shared MLP: f32 [T, H]
-    uint64_t tiles;      // prefill GEMM: i32 tile list
+    uint64_t tiles;      // prefill GEMM and lp_mid.hip: i32 tile list
     uint64_t actimg;     // prefill GEMM: [T*k] fp16 images of act rows (himage_bytes(I) each)
     uint64_t xexp;       // prefill GEMM: i32 [T], token t's image exponent in xf
     uint64_t disp;       // multi-block dispatch: i32 [nb][E] counts, [nb][E] first positions, [E] entries
@@ -361,6 +361,7 @@ LPK_HD constexpr int shared_entries(int T) { return T <= 64 ? (T + kEntryToks - 
 
 constexpr int kImgF16 = 1;     // RouteArgs::make_xf bits
 constexpr int kImgDigits = 2;
+constexpr int kImgF16Lo = 4;   // with kImgF16: the lo images too, after the T hi images (T > 64 only)
 
 struct RouteArgs {
     LayerView L;
@@ -370,6 +371,9 @@ struct RouteArgs {
     int32_t make_xf;     // router: also write images of x: kImgF16 into W.xf (+ W.xexp), kImgDigits into W.xd
     uint64_t sync;       // fused routing: kSyncWords arrival counters, zero between launches
     int32_t tok_block;   // fused routing: tokens per block (grid y = ceil(T / tok_block))
+    int32_t tile_tokens; // batches above 64 tokens: tokens per entry of the tile list (0: none)
+    uint64_t tiles;      // the list: (entry << 16) | block, at most max_tiles of them, their number in meta[2]
+    int32_t max_tiles;
     int32_t pad0;
 };
 
@@ -460,6 +464,37 @@ struct GemmArgs {
     int32_t T;
     int32_t max_tiles;
     int32_t nblocks;     // weight-row blocks per tile row
+    int32_t pad0;
+};
+
+// Batches between decode and prefill (lp_mid.hip): blocks of up to kMidToks
+// tokens of one expert (16 per MFMA tile); 128 act columns (kActChunk) or
+// kMidRows rows of down per workgroup of four waves.
+constexpr int kMidToks = 32;
+constexpr int kMidMinPairsPerExpert = 5;
+constexpr int kMidRows = 256;
+// LDS: the scales of 64 sub-groups of each of the 256 weight rows (8 bytes of
+// pad: 16 rows' 8-byte reads then cover the banks), two slots of the token
+// tiles' rows of a stage (128 columns, hi and lo; 16 pieces of 16 tokens and a
+// pad each), then the tokens' exponents.
+constexpr int kMidScaleRow = 136;
+constexpr int kMidScaleBytes = 256 * kMidScaleRow;
+constexpr int kMidBlk = 16 * 17;  // 16-byte words of one token tile's hi or lo rows
+constexpr int kMidEpRow = 20;     // floats per row of the gate/up epilogue's tiles (16 tokens, a pad), in the slots
+constexpr int kMidExOff = kMidScaleBytes + 2 * 2 * 2 * kMidBlk * 16;
+constexpr int kMidLds = kMidExOff + 4 * kMidToks;
+static_assert(256 * kMidEpRow * 4 <= 2 * 2 * 2 * kMidBlk * 16, "the epilogue fits the slots");
+
+struct MidArgs {
+    LayerView L;         // inter, group and regions of the matrices taken (routed or shared)
+    Workspace W;         // et, perm, meta, xexp
+    uint64_t img;        // token images (hi): gate/up by token, down by dispatch position
+    uint64_t img_stride; // bytes from one row's image to the next
+    uint64_t lo_off;     // bytes from a row's hi image to its lo image
+    uint64_t out;        // gate/up: act images, hi and lo per dispatch position; down: y f32
+    uint64_t exps;       // act exponents i32 [position][inter / 32]
+    uint64_t tiles;      // (entry << 16) | block of kMidToks tokens, meta[2] of them; 0: entry 0's blocks
+    int32_t chunks;      // workgroups per block (grid = blocks x chunks)
     int32_t pad0;
 };
 

@@ -67,7 +67,6 @@ enum Fn {
     kTopkDispatch,
     kExpfWave,
     kResolve,
-    kGemmTiles,
     kGemmGateup,
     kGemmDown,
     kDispCount,
@@ -119,6 +118,10 @@ enum Fn {
     kAttnBlockG4,
     kAttnBlockG8,
     kAttnBlockG16,
+    kMidGateup,
+    kMidGateupRs,
+    kMidDown,
+    kMidDownRs,
     kNumFns
 };
 
@@ -137,8 +140,7 @@ const FnSpec kSpecs[kNumFns] = {
     {"lp_moe.hsaco", "lp_moe_combine"},    {"lp_moe.hsaco", "lp_moe_ximage"},
     {"lp_moe.hsaco", "lp_moe_topk_dispatch"}, {"lp_basic.hsaco", "lp_expf_wave"},
     {"lp_moe.hsaco", "lp_moe_resolve"},
-    {"lp_gemm.hsaco", "lp_gemm_tiles"},    {"lp_gemm.hsaco", "lp_gemm_gateup"},
-    {"lp_gemm.hsaco", "lp_gemm_down"},
+    {"lp_gemm.hsaco", "lp_gemm_gateup"},   {"lp_gemm.hsaco", "lp_gemm_down"},
     {"lp_moe.hsaco", "lp_moe_disp_count"}, {"lp_moe.hsaco", "lp_moe_disp_scan"},
     {"lp_moe.hsaco", "lp_moe_disp_scatter"}, {"lp_gemm.hsaco", "lp_gemm_router"},
     {"lp_moe.hsaco", "lp_moe_dispatch"},   {"lp_moe.hsaco", "lp_moe_route_fused"},
@@ -166,11 +168,13 @@ const FnSpec kSpecs[kNumFns] = {
     {"lp_step.hsaco", "lp_attn_block_g1"}, {"lp_step.hsaco", "lp_attn_block_g2"},
     {"lp_step.hsaco", "lp_attn_block_g4"}, {"lp_step.hsaco", "lp_attn_block_g8"},
     {"lp_step.hsaco", "lp_attn_block_g16"},
+    {"lp_mid.hsaco", "lp_mid_gateup"},       {"lp_mid.hsaco", "lp_mid_gateup_rs"},
+    {"lp_mid.hsaco", "lp_mid_down"},         {"lp_mid.hsaco", "lp_mid_down_rs"},
 };
 
 const char* const kModules[] = {"lp_basic.hsaco", "lp_moe.hsaco", "lp_gemm.hsaco", "lp_attn.hsaco",
-                                "lp_step.hsaco"};
-constexpr int kNumModules = 5;
+                                "lp_step.hsaco", "lp_mid.hsaco"};
+constexpr int kNumModules = 6;
 
 std::string library_dir() {
     Dl_info info;
@@ -1003,16 +1007,37 @@ static bool use_gemm(const lp_moe_layer_desc* d, int T) {
            act_chunks(d->inter) <= kGemmMaxChunks;
 }
 
-// The images of x a layer's expert kernels read: fp16 images for the prefill
-// GEMM, digit images for the grouped kernels (every shared MLP included).
-static int image_kinds(const lp_moe_layer_desc* d, int T) {
-    const bool gemm = use_gemm(d, T);
-    return (gemm ? kImgF16 : 0) | (!gemm || d->shared_blob ? kImgDigits : 0);
+// Batches between decode and prefill (lp_mid.hip): the routed experts once
+// they average kMidMinPairsPerExpert pairs (a 16-token tile then holds enough
+// tokens to beat the decode kernels' passes of four), the shared MLP of every
+// batch above the decode sizes (all T tokens in one entry).
+static bool use_mid(const lp_moe_layer_desc* d, int T) {
+    const long pairs = (long)T * d->top_k;
+    return T > kTopkDispatchMaxT && !use_gemm(d, T) && d->slot_span < (1ull << 31) &&
+           pairs >= (long)kMidMinPairsPerExpert * std::min<long>(d->experts, pairs);
 }
 
-static int gemm_max_tiles(const lp_moe_layer_desc* d, int T) {
+static bool use_mid_shared(const lp_moe_layer_desc* d, int T) { return T > kTopkDispatchMaxT && d->shared_blob; }
+
+// The images of x a layer's expert kernels read: fp16 images for the prefill
+// GEMM, hi + lo ones for lp_mid.hip, digit images for the grouped kernels.
+static int image_kinds(const lp_moe_layer_desc* d, int T) {
+    const bool gemm = use_gemm(d, T), mid = use_mid(d, T), mid_sh = use_mid_shared(d, T);
+    return (gemm || mid || mid_sh ? kImgF16 : 0) | (mid || mid_sh ? kImgF16Lo : 0) |
+           ((!gemm && !mid) || (d->shared_blob && !mid_sh) ? kImgDigits : 0);
+}
+
+static uint64_t mid_exps_bytes(uint64_t rows, int inter) { return align256(rows * (uint64_t)(inter / 32) * 4); }
+
+// The tile list of a batch above the decode sizes: blocks of this many tokens
+// of each routed expert (0: no list), at most max_tiles of them.
+static int tile_tokens(const lp_moe_layer_desc* d, int T) {
+    return T <= kTopkDispatchMaxT ? 0 : use_gemm(d, T) ? kGemmBM : use_mid(d, T) ? kMidToks : 0;
+}
+
+static int max_tiles(const lp_moe_layer_desc* d, int T, int tokens) {
     const int pairs = T * d->top_k;
-    return pairs / kGemmBM + std::min(d->experts, pairs) + 1;
+    return pairs / tokens + std::min(d->experts, pairs) + 1;
 }
 
 // Workgroups of a GEMM launch: a multiple of kXcds covering every possible
@@ -1042,20 +1067,25 @@ int lp_moe_ws_layout_get(const lp_moe_layer_desc* d, int T, lp_moe_ws_layout* ou
     out->uniq = take(E * 4);
     out->meta = take(64);
     out->et = take(E * sizeof(ExpertEntry));
-    // the prefill GEMM writes act as fp16 images (actimg), their chunk exponents here
-    out->act = take(use_gemm(d, T) ? t * k * (uint64_t)act_chunks((int)I) * 4 : t * k * I * 4);
+    // the prefill GEMM and lp_mid.hip write act as fp16 images (actimg), their exponents here
+    const bool mid = use_mid(d, T), mid_sh = use_mid_shared(d, T);
+    const int kinds = image_kinds(d, T);
+    out->act = take(use_gemm(d, T) ? t * k * (uint64_t)act_chunks((int)I) * 4
+                    : mid          ? mid_exps_bytes(t * k, (int)I)
+                                   : t * k * I * 4);
     out->y = take(t * k * H * 4);
-    out->xf = take(use_gemm(d, T) ? t * (uint64_t)himage_bytes((int)H) : 0);
+    out->xf = take(kinds & kImgF16 ? t * (uint64_t)himage_bytes((int)H) * (kinds & kImgF16Lo ? 2 : 1) : 0);
     out->xd = take(t * (uint64_t)dimage_bytes((int)H));
     const bool sh = d->shared_blob != 0;
     const uint64_t Is = sh ? (uint64_t)d->shared_inter : 0;
     out->sh_et = take(sh ? (uint64_t)shared_entries(T) * sizeof(ExpertEntry) : 0);
     out->sh_perm = take(sh ? t * 4 : 0);
-    out->sh_act = take(t * Is * 4);
+    out->sh_act = take(mid_sh ? mid_exps_bytes(t, (int)Is) + t * 2 * (uint64_t)himage_bytes((int)Is) : t * Is * 4);
     out->sh_y = take(sh ? t * H * 4 : 0);
     const bool gemm = use_gemm(d, T);
-    out->tiles = take(gemm ? (uint64_t)gemm_max_tiles(d, T) * 4 : 0);
-    out->actimg = take(gemm ? t * k * (uint64_t)himage_bytes((int)I) : 0);
+    const int tt = tile_tokens(d, T);
+    out->tiles = take(tt ? (uint64_t)max_tiles(d, T, tt) * 4 : 0);
+    out->actimg = take(gemm || mid ? t * k * (uint64_t)himage_bytes((int)I) * (mid ? 2 : 1) : 0);
     out->xexp = take(t * 4);
     out->disp = take(T > kTopkDispatchMaxT ? (2 * ((t + kDispTok - 1) / kDispTok) + 1) * E * 4 : 0);
     out->total = o;
@@ -1188,6 +1218,13 @@ static int check_ws(const lp_moe_layer_desc* d, int T, uint64_t ws, uint64_t ws_
     return LP_OK;
 }
 
+// The tile list the dispatch of a batch above 64 tokens writes.
+static void set_tiles(const lp_moe_layer_desc* d, RouteArgs& ra) {
+    ra.tile_tokens = tile_tokens(d, ra.T);
+    ra.tiles = ra.W.tiles;
+    ra.max_tiles = ra.tile_tokens ? max_tiles(d, ra.T, ra.tile_tokens) : 0;
+}
+
 static int route_tail(lp_ctx* c, const RouteArgs& ra, lp_stream s) {
     const int T = ra.T;
     // up to kTopkFusedMaxT tokens: one workgroup does both (one token per
@@ -1222,6 +1259,7 @@ int lp_moe_route(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t x, int T, uint6
     ra.x = x;
     ra.T = T;
     ra.make_xf = image_kinds(d, T);
+    set_tiles(d, ra);
     if (T > kTopkDispatchMaxT) {
         // large batch: the MFMA router, then the images of x on their own
         dim3 g((unsigned)((T + 15) / 16), (unsigned)((d->experts + 31) / 32));
@@ -1256,6 +1294,7 @@ int lp_moe_route_logits(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t logits, 
     RouteArgs ra{};
     fill_views(d, ws, T, &ra.L, &ra.W);
     ra.T = T;
+    set_tiles(d, ra);
     if (logits != ra.W.logits)
         HIPCHK(hipMemcpyAsync(reinterpret_cast<void*>(ra.W.logits), reinterpret_cast<void*>(logits),
                               (size_t)T * d->experts * 4, hipMemcpyDeviceToDevice, (hipStream_t)s));
@@ -1419,6 +1458,50 @@ static int shared_ffn(lp_ctx* c, const lp_moe_layer_desc* d, const GroupedArgs& 
     return grouped_ffn(c, gs, shared_entries(T), false, s, with_down);
 }
 
+// Gate/up and down through lp_mid.hip for `blocks` blocks of kMidToks tokens
+// (at most: the tile list's count decides; tiles 0: all of entry 0) of ga's
+// entries: exps and actimg hold act's exponents and hi + lo images by
+// dispatch position.
+static int mid_ffn(lp_ctx* c, const GroupedArgs& ga, int blocks, uint64_t tiles, uint64_t exps, uint64_t actimg,
+                   lp_stream s) {
+    MidArgs m{};
+    m.L = ga.L;
+    m.W = ga.W;
+    m.exps = exps;
+    m.tiles = tiles;
+    const int H = ga.L.hidden, I = ga.L.inter;
+    auto vec = [&](int cols) { return ga.L.group == 32 && (cols / 32) % 4 == 0; };
+    m.img = ga.W.xf;
+    m.img_stride = (uint64_t)himage_bytes(H);
+    m.lo_off = (uint64_t)ga.T * himage_bytes(H);
+    m.out = actimg;
+    m.chunks = act_chunks(I);
+    if (int r = launch(c, vec(H) ? kMidGateup : kMidGateupRs, dim3((unsigned)(blocks * m.chunks)), dim3(256), kMidLds, s,
+                       m))
+        return r;
+    m.img = actimg;
+    m.img_stride = 2 * (uint64_t)himage_bytes(I);
+    m.lo_off = (uint64_t)himage_bytes(I);
+    m.out = ga.W.y;
+    m.chunks = (H + kMidRows - 1) / kMidRows;
+    return launch(c, vec(I) ? kMidDown : kMidDownRs, dim3((unsigned)(blocks * m.chunks)), dim3(256), kMidLds, s, m);
+}
+
+// The shared MLP of a batch above the decode sizes: one entry of all T tokens.
+static int mid_shared_ffn(lp_ctx* c, const lp_moe_layer_desc* d, const GroupedArgs& ga, int T, lp_stream s) {
+    GroupedArgs gs = ga;
+    gs.L.inter = d->shared_inter;
+    gs.L.group = d->shared_group;
+    gs.L.gate_off = d->sh_gate_off;
+    gs.L.up_off = d->sh_up_off;
+    gs.L.down_off = d->sh_down_off;
+    gs.L.top_k = 1;
+    gs.W.et = ga.W.sh_et;
+    gs.W.perm = ga.W.sh_perm;
+    gs.W.y = ga.W.sh_y;
+    return mid_ffn(c, gs, (T + kMidToks - 1) / kMidToks, 0, ga.W.sh_act, ga.W.sh_act + mid_exps_bytes((uint64_t)T, d->shared_inter), s);
+}
+
 // The grouped expert kernels and the combine; the fragment images of x are
 // written first unless the router kernel of lp_moe_forward already did.
 // wave_n > 0: only the routed experts uniq[wave_u0, wave_u0 + wave_n) (one
@@ -1482,8 +1565,7 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         gm.W = ga.W;
         gm.T = T;
         gm.tiles = ga.W.tiles;
-        gm.max_tiles = gemm_max_tiles(d, T);
-        if (int r = launch(c, kGemmTiles, dim3(1), dim3(256), 0, s, gm)) return r;
+        gm.max_tiles = max_tiles(d, T, kGemmBM);
         // gate/up writes act as the down GEMM's fp16 images (+ chunk exponents in W.act)
         gm.a_img = ga.W.xf;
         gm.out = ga.W.actimg;
@@ -1495,6 +1577,8 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         gm.nblocks = (d->hidden + kGemmBN - 1) / kGemmBN;
         if (int r = launch(c, kGemmDown, dim3(gemm_grid(gm)), dim3(kGemmWaves * 64), 0, s, gm))
             return r;
+    } else if (!wave && use_mid(d, T)) {
+        if (int r = mid_ffn(c, ga, max_tiles(d, T, kMidToks), ga.W.tiles, ga.W.act, ga.W.actimg, s)) return r;
     } else {
         // one token: down and combine in one launch (after the shared MLP,
         // whose row it adds)
@@ -1504,7 +1588,8 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
                           (size_t)comb_lds(d->inter, Si, sl) <= c->max_lds;
         // the shared MLP's gate/up rides on the routed balanced launch when
         // the groups agree (sh_gu: it did)
-        const int shm = !wave && d->shared_blob && d->shared_group == d->group ? shared_entries(T) : 0;
+        const int shm =
+            !wave && d->shared_blob && d->shared_group == d->group && !use_mid_shared(d, T) ? shared_entries(T) : 0;
         if (int r = grouped_ffn(c, ga, maxu, true, s, !comb, shm, &sh_gu)) return r;
         if (comb) {
             const Fn f = !sl ? kDownCombRs : Si <= 8 ? kDownComb : kDownComb16;
@@ -1524,8 +1609,11 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
                           lds, s, ga);
         }
     }
-    if (d->shared_blob)
+    if (use_mid_shared(d, T)) {
+        if (int r = mid_shared_ffn(c, d, ga, T, s)) return r;
+    } else if (d->shared_blob) {
         if (int r = shared_ffn(c, d, ga, T, s, true, !sh_gu)) return r;
+    }
     return launch(c, kCombine, dim3((unsigned)((d->hidden + 1023) / 1024), (unsigned)T), dim3(256), 0,
                   s, ga);
 }
