@@ -471,7 +471,7 @@ struct GemmArgs {
 // tokens of one expert (16 per MFMA tile); 128 act columns (kActChunk) or
 // kMidRows rows of down per workgroup of four waves.
 constexpr int kMidToks = 32;
-constexpr int kMidMinPairsPerExpert = 5;
+constexpr int kMidMinPairsPerExpert = 6;
 constexpr int kMidRows = 256;
 // LDS: the scales of 64 sub-groups of each of the 256 weight rows (8 bytes of
 // pad: 16 rows' 8-byte reads then cover the banks), two slots of the token

@@ -1007,14 +1007,23 @@ static bool use_gemm(const lp_moe_layer_desc* d, int T) {
            act_chunks(d->inter) <= kGemmMaxChunks;
 }
 
-// Batches between decode and prefill (lp_mid.hip): the routed experts once
-// they average kMidMinPairsPerExpert pairs (a 16-token tile then holds enough
-// tokens to beat the decode kernels' passes of four), the shared MLP of every
-// batch above the decode sizes (all T tokens in one entry).
+// Batches between decode and prefill: the routed experts of more than 64
+// tokens go through lp_mid.hip unless the balanced decode kernels take both
+// projections (one chunk of K, no more token groups of four than the card's
+// 256 CUs) and the experts average fewer than kMidMinPairsPerExpert pairs:
+// those re-read no weights for so few tokens (H 2048 / I 768 / 128 experts /
+// top 8: 80 tokens 56.6 + 32.0 us balanced, 63.4 + 39.0 here; past the 256
+// groups the alternative is the one-shot kernels, 81 tokens 104.0 + 56.9,
+// 62.9 + 39.2 here; H 4096 / I 1536, 65 tokens: 429.5 + 145.0 one-shot,
+// 193.4 + 102.6 here).  The shared MLP of every batch above the decode sizes
+// (all T tokens in one entry) goes there too.
 static bool use_mid(const lp_moe_layer_desc* d, int T) {
-    const long pairs = (long)T * d->top_k;
+    const long pairs = (long)T * d->top_k, maxu = std::min<long>(d->experts, pairs);
+    const bool balanced = frag_ngp(d->hidden) <= 4 * kGateupChunk && frag_ngp(d->inter) <= 4 * 8 &&
+                          scales_in_lds(d->group, d->inter) && maxu <= kBalMaxU &&
+                          (pairs + (kBalToks - 1) * maxu) / kBalToks <= 256;
     return T > kTopkDispatchMaxT && !use_gemm(d, T) && d->slot_span < (1ull << 31) &&
-           pairs >= (long)kMidMinPairsPerExpert * std::min<long>(d->experts, pairs);
+           (!balanced || pairs >= kMidMinPairsPerExpert * maxu);
 }
 
 static bool use_mid_shared(const lp_moe_layer_desc* d, int T) { return T > kTopkDispatchMaxT && d->shared_blob; }

@@ -51,14 +51,16 @@ def _check(cuda, L, T, seed, logits=None, blobs=None, scale=1.0, want_err=0):
 
 # widths around the stages of 128 columns and the 128-column / 256-row blocks:
 # one sub-group past, a lone one, rows short of a block; every group size; a
-# token count just past the decode sizes, averages from 5 to just below 16
+# token count just past the decode sizes; averages from 2 (rows wider than the
+# balanced kernels take, or more token groups than CUs) to just below 16
 @pytest.mark.parametrize("H,I,E,k,group,T", [
     (2048, 768, 128, 8, 32, 81), (2048, 768, 128, 8, 32, 203), (2048, 1408, 64, 6, 32, 100), (160, 96, 16, 2, 32, 65),
     (384, 32, 32, 4, 32, 100), (288, 544, 24, 3, 32, 127), (192, 128, 16, 2, 64, 90), (512, 384, 10, 1, 128, 77),
-    (4096, 256, 16, 2, 32, 66), (128, 128, 12, 1, 32, 191)])
+    (4096, 256, 16, 2, 32, 66), (128, 128, 12, 1, 32, 191), (2176, 64, 32, 1, 32, 66), (64, 64, 300, 4, 32, 70),
+    (128, 128, 32, 2, 32, 96), (128, 128, 32, 2, 32, 95)])
 def test_mid_layer(cuda, H, I, E, k, group, T):
     L = DeviceLayer(cuda, H=H, I=I, E=E, k=k, group=group, seed=H + I)
-    assert T > 64 and 5 * E <= T * k < 16 * E, "between decode and the prefill GEMM"
+    assert T > 64 and T * k < 16 * E, "between decode and the prefill GEMM"
     _check(cuda, L, T, T)
     L.free()
 
