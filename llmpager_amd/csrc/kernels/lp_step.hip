@@ -230,7 +230,7 @@ LP_GEMV_KERNELS(8)
 // ---------------------------------------------------------------------------
 // Fused GQA decode attention for head_dim 128 and G query heads per KV head
 // (the reference's rmsnorm per head, rope, kv_append and attn_decode_f16kv,
-// decode.rs:283-294).  Grid (splits, kv_heads), 4 waves.  Workgroup (s, g):
+// decode.rs:283-294).  4 waves; workgroup s + splits g is split s of KV head g:
 //
 //   prologue  the G query heads of KV head g: RMSNorm with q_norm, NeoX RoPE
 //             at pos (decode.cu:17-41, 145-167), into LDS; the split holding
@@ -249,9 +249,16 @@ LP_GEMV_KERNELS(8)
 //             probabilities read from LDS.  Row pos comes from LDS, not from
 //             the cache being written.
 //   merge     the four waves' states in LDS; one split writes the output, more
-//             write partial records {max, sum, acc[128]} to the scratch and
-//             the last of them to arrive (a counter per KV head) merges them,
-//             its record loads issued in one burst.
+//             write partial records {max, sum, acc[128]} to the scratch.  Up to
+//             kAttnLastMerge splits: the last of a KV head to arrive (a counter
+//             per KV head) merges its records, loads in bursts of 16 splits.
+//             More: one workgroup per query head, after the splits' in the
+//             grid, waits for its KV head's count and merges that head's, all
+//             loads in one burst; waiting costs a poll that the last arrival
+//             does not pay (24 splits at 32 heads on 4 KV heads: the block
+//             19.6 us merged by the last arrival, 20.1 by heads), reading G
+//             heads in three or more rounds costs more (13,002 positions: 28.7
+//             us with at most 32 splits and the last arrival, 25.9 with 64).
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -287,11 +294,12 @@ __device__ __forceinline__ float row16_max(float v) {
     return fmaxf(v, dpp<0x128>(v));
 }
 
-// The attention output leaves by agent-scope stores when another workgroup
-// of the launch reads it (done != null); the workgroup that completes a KV
-// head's output then adds one to *done.
+// One split of a KV head.  The attention output (one split) leaves by
+// agent-scope stores when another workgroup of the launch reads it (done !=
+// null), and *done counts the KV heads complete; with more splits the records
+// do, and the KV head's own counter.
 template <int G>
-__device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, int g, int* done) {
+__device__ __forceinline__ void attn_split_body(const AttnFusedArgs& a, int sp, int g, int* done) {
     constexpr int STEPS = kHd / 32;
     __shared__ __align__(16) float qf[G][kHd];
     __shared__ __align__(16) uint4 qb[2][STEPS][64];
@@ -300,7 +308,7 @@ __device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, 
     __shared__ float al[4][16];                     // wave, head: this chunk's rescale
     __shared__ __align__(16) float wacc[4][G][kHd];
     __shared__ float wm[4][16], wl[4][16];
-    __shared__ float mw[16 * kAttnFusedMaxSplits];
+    __shared__ float mw[16 * kAttnLastMerge];
     __shared__ int flag;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const int n = lane & 15, kb = lane >> 4;
@@ -539,6 +547,10 @@ __device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, 
         return;
     }
     int* cnt = reinterpret_cast<int*>(a.sync) + kStepSyncAttn + kSyncStride * g;
+    if (a.splits > kAttnLastMerge) {  // a workgroup per query head merges (attn_merge_body)
+        signal_count(cnt);
+        return;
+    }
     if (arrival_order(cnt, a.splits, &flag) != a.splits - 1) return;
     // ---- the last split of head group g merges the records.  They were
     // written in this launch with agent-scope stores and nothing on this XCD
@@ -585,7 +597,7 @@ __device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, 
                 const float e = s < S ? exp_hw(mr[p] - M) : 0.0f;
                 float den = row16_sum(e * lr[p]);
                 den += shfl_xor(den, 16);
-                if (hh < G && s < S) mw[hh * kAttnFusedMaxSplits + s] = e / den;
+                if (hh < G && s < S) mw[hh * kAttnLastMerge + s] = e / den;
             }
             __syncthreads();
         }
@@ -595,7 +607,7 @@ __device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, 
             for (int i = 0; i < kOut; ++i) {
                 const int hh = (tid + 256 * i) >> 5;
                 if (s0 + k < S && hh < G) {
-                    const float wt = mw[hh * kAttnFusedMaxSplits + s0 + k];
+                    const float wt = mw[hh * kAttnLastMerge + s0 + k];
                     num[i].x = __builtin_fmaf(wt, v[k][i].x, num[i].x);
                     num[i].y = __builtin_fmaf(wt, v[k][i].y, num[i].y);
                     num[i].z = __builtin_fmaf(wt, v[k][i].z, num[i].z);
@@ -621,11 +633,90 @@ __device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a, int sp, 
     if (done) signal_count(done);
 }
 
+// The merge of query head `head`'s records, once its KV head's splits are
+// complete.  They were written in this launch with agent-scope stores and
+// nothing on this XCD has read them since the launch began, so plain loads
+// see them: the {max, sum} pairs (lane s of each wave holding split s) and
+// the accumulators (32 threads x 16 bytes per record, eight records at a
+// time, all of them before the first is used).
+__device__ __forceinline__ void attn_merge_body(const AttnFusedArgs& a, int head, int group, bool agent) {
+    __shared__ __align__(16) float4 part[8][32];
+    __shared__ float mw[kAttnFusedMaxSplits];
+    static_assert(kAttnFusedMaxSplits == 64, "one split per lane");
+    int* sync = reinterpret_cast<int*>(a.sync);
+    const int S = a.splits, tid = threadIdx.x, lane = lane_id();
+    wait_count(sync + kStepSyncAttn + kSyncStride * (head / group), S, sync + kStepSyncErr, a.spin_max);
+    const uint64_t rec = a.scratch + (uint64_t)head * (uint32_t)a.scratch_stride * 4u;
+    constexpr uint32_t kRecBytes = kAttnFusedRec * 4;
+    const float2 ml = *gptr<float2>(rec + (uint64_t)min(lane, S - 1) * kRecBytes + kHd * 4);
+    const int r = tid >> 5, d4 = tid & 31;
+    float4 v[kAttnFusedMaxSplits / 8];
+#pragma unroll
+    for (int k = 0; k < kAttnFusedMaxSplits / 8; ++k)  // past the last: that one again, weight zero
+        v[k] = *gptr<float4>(rec + (uint64_t)min(8 * k + r, S - 1) * kRecBytes + 16u * (uint32_t)d4);
+    float M = lane < S ? ml.x : -INFINITY;
+    M = row16_max(M);
+    M = fmaxf(M, shfl_xor(M, 16));
+    M = fmaxf(M, shfl_xor(M, 32));
+    const float e = lane < S ? exp_hw(ml.x - M) : 0.0f;
+    float den = row16_sum(lane < S ? e * ml.y : 0.0f);
+    den += shfl_xor(den, 16);
+    den += shfl_xor(den, 32);
+    if (tid < 64) mw[lane] = e / den;
+    __syncthreads();
+    float4 num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int k = 0; k < kAttnFusedMaxSplits / 8; ++k) {
+        if (8 * k + r < S) {
+            const float w = mw[8 * k + r];
+            num.x = __builtin_fmaf(w, v[k].x, num.x);
+            num.y = __builtin_fmaf(w, v[k].y, num.y);
+            num.z = __builtin_fmaf(w, v[k].z, num.z);
+            num.w = __builtin_fmaf(w, v[k].w, num.w);
+        }
+    }
+    part[r][d4] = num;
+    __syncthreads();
+    if (tid < kHd) {
+        const float* p = reinterpret_cast<const float*>(part) + tid;
+        float t = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t += p[q * kHd];
+        float* out = reinterpret_cast<float*>(a.out) + (size_t)head * kHd + tid;
+        if (agent)
+            agent_store(out, t);
+        else
+            *out = t;
+    }
+}
+
+// Every KV head's count back to zero, once all of its waits have passed.
+__device__ __forceinline__ void attn_counts_clear(int* sync, int kv_heads) {
+    if ((int)threadIdx.x < kv_heads) agent_store(sync + kStepSyncAttn + kSyncStride * threadIdx.x, 0);
+}
+
+// lp_attn_fused: workgroups [0, splits kv_heads) the splits, then (more than
+// kAttnLastMerge splits) one per query head, the last of which to finish
+// clears the counts.
+template <int G>
+__device__ __forceinline__ void attn_fused_body(const AttnFusedArgs& a) {
+    const int n_attn = a.splits * a.kv_heads;
+    if ((int)blockIdx.x < n_attn) {
+        attn_split_body<G>(a, blockIdx.x % a.splits, blockIdx.x / a.splits, nullptr);
+        return;
+    }
+    __shared__ int flag;
+    attn_merge_body(a, (int)blockIdx.x - n_attn, G, false);
+    int* sync = reinterpret_cast<int*>(a.sync);
+    const int heads = G * a.kv_heads;
+    if (arrival_order(sync + kStepSyncDone, heads, &flag) == heads - 1) attn_counts_clear(sync, a.kv_heads);
+}
+
 }  // namespace
 
 #define LP_ATTN_FUSED(G)                                                                             \
     extern "C" __global__ void __launch_bounds__(256) lp_attn_fused_g##G(const AttnFusedArgs a) {  \
-        attn_fused_body<G>(a, blockIdx.x, blockIdx.y, nullptr);                                      \
+        attn_fused_body<G>(a);                                                                       \
     }
 LP_ATTN_FUSED(1)
 LP_ATTN_FUSED(2)
@@ -636,12 +727,12 @@ LP_ATTN_FUSED(16)
 
 // ---------------------------------------------------------------------------
 // The attention block's tail in one launch: lp_attn_fused on workgroups
-// [0, n_attn) (split s of KV head g at s + splits g), then the o projection,
-// the residual add and the post-attention norm (lp_gemv_add_rmsnorm) on the
+// [0, n_attn) (its splits, then its merges), then the o projection, the
+// residual add and the post-attention norm (lp_gemv_add_rmsnorm) on the
 // workgroups after them.  Those start by loading their rows of W_o, which do
-// not depend on the attention, then wait for the attention's KV heads to be
-// complete (a counter) and read its output with agent-scope loads.  The last
-// of them resets the counter.
+// not depend on the attention, then wait for its KV heads (query heads, where
+// those are merged one by one) to be complete (a counter) and read its output.  Every wait is for
+// workgroups of lower index.  The last of them resets the counters.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -651,8 +742,14 @@ template <int G>
 __device__ __forceinline__ void attn_block_body(const AttnBlockArgs& b) {
     const AttnFusedArgs& a = b.at;
     int* sync = reinterpret_cast<int*>(a.sync);
+    const int n_split = a.splits * a.kv_heads;
+    if ((int)blockIdx.x < n_split) {
+        attn_split_body<G>(a, blockIdx.x % a.splits, blockIdx.x / a.splits, sync + kStepSyncDone);
+        return;
+    }
     if ((int)blockIdx.x < b.n_attn) {
-        attn_fused_body<G>(a, blockIdx.x % a.splits, blockIdx.x / a.splits, sync + kStepSyncDone);
+        attn_merge_body(a, (int)blockIdx.x - n_split, G, true);
+        signal_count(sync + kStepSyncDone);
         return;
     }
     __shared__ float red[4];
@@ -667,7 +764,7 @@ __device__ __forceinline__ void attn_block_body(const AttnBlockArgs& b) {
     float hr[kBlockRowsPerWave];
 #pragma unroll
     for (int r = 0; r < kBlockRowsPerWave; ++r) hr[r] = r0 + r < b.rows ? reinterpret_cast<const float*>(b.h)[r0 + r] : 0.0f;
-    wait_count(sync + kStepSyncDone, a.kv_heads, sync + kStepSyncErr, b.spin_max);
+    wait_count(sync + kStepSyncDone, a.splits <= kAttnLastMerge ? a.kv_heads : G * a.kv_heads, sync + kStepSyncErr, a.spin_max);
     // the attention output: written in this launch with agent-scope stores,
     // and nothing on this XCD read it before they completed, so plain loads
     // see it
@@ -681,8 +778,9 @@ __device__ __forceinline__ void attn_block_body(const AttnBlockArgs& b) {
     }
     const int n_o = (int)gridDim.x - b.n_attn;
     if (arrival_order(sync + kStepSyncGemv, n_o, &flag) != n_o - 1) return;
-    // every workgroup has passed its wait: the counter starts the next launch at zero
+    // every workgroup has passed its wait: the counters start the next launch at zero
     if (threadIdx.x == 0) agent_store(sync + kStepSyncDone, 0);
+    if (a.splits > kAttnLastMerge) attn_counts_clear(sync, a.kv_heads);
     constexpr int kPer = kFusedGemvMaxRows / 256;
     const float* ln = reinterpret_cast<const float*>(b.ln);
     float hv[kPer], gv[kPer];

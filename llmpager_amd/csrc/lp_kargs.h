@@ -30,7 +30,7 @@ constexpr int kSyncStride = 32;        // words between arrival counters (one 12
 constexpr int kAttnFusedMaxKvHeads = 16;
 constexpr int kStepSyncAttn = 17 * kSyncStride;
 constexpr int kStepSyncGemv = kStepSyncAttn + kAttnFusedMaxKvHeads * kSyncStride;
-constexpr int kStepSyncDone = kStepSyncGemv + kSyncStride;  // lp_attn_block: KV heads complete
+constexpr int kStepSyncDone = kStepSyncGemv + kSyncStride;  // KV (or query) heads complete
 constexpr int kStepSyncErr = kStepSyncDone + kSyncStride;   // waits that gave up (lp_step_errors_sync)
 constexpr int kSyncWords = kStepSyncErr + kSyncStride;
 constexpr int kMaxTopK = 16;           // largest top_k the device router accepts
@@ -152,24 +152,26 @@ struct GemvAddRmsNormArgs {
 // positions per split; partial records {acc[128], max, sum, 2 unused} at
 // scratch + head * scratch_stride + split * kAttnFusedRec floats when
 // splits > 1.
-constexpr int kAttnFusedMaxSplits = 32;
+constexpr int kAttnFusedMaxSplits = 64;
+constexpr int kAttnLastMerge = 32;  // splits a KV head's last arrival merges; above, a workgroup per query head
 constexpr int kAttnFusedRec = 128 + 4;
 struct AttnFusedArgs {
     uint64_t q, k, v, q_norm, k_norm;
     uint64_t kcache, vcache, out, scratch, sync;
     int32_t kv_heads, pos, max_seq, splits, cps, scratch_stride;
     float eps, rope_base, scale;
-    int32_t pad0;
+    int32_t spin_max;
 };
 
-// lp_attn_fused on workgroups [0, n_attn) (at.out the attention output),
+// lp_attn_fused on workgroups [0, n_attn) (at.out the attention output; the
+// splits, then above kAttnLastMerge splits a merge per query head),
 // then h[rows] += W_o . out (W_o bf16 [rows, cols]) and hn = rmsnorm(h, ln)
 // on the workgroups after them
 constexpr int kStepSpinMax = 1 << 15;  // polls (about a microsecond each) before the wait gives up
 struct AttnBlockArgs {
     AttnFusedArgs at;
     uint64_t wo, h, ln, hn;
-    int32_t rows, cols, n_attn, spin_max;
+    int32_t rows, cols, n_attn, pad0;
 };
 
 struct AddArgs {                    // kernels.rs:239-250

@@ -937,7 +937,9 @@ static int attn_fused_plan(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64
     // records are read 16 bytes at a time: each head's row of the scratch
     // starts at a multiple of 4 floats
     const int stride = max_seq & ~3;
-    const int by_scratch = stride / kAttnFusedRec;
+    // (and a head's last record must not share a cache line with the next
+    // head's first: they are read in one launch at different times)
+    const int by_scratch = (stride - 32) / kAttnFusedRec;
     int splits = std::min(chunks, std::min(kAttnFusedMaxSplits, by_scratch));
     if (splits < 1) splits = 1;
     const int cps = (chunks + splits - 1) / splits;
@@ -950,6 +952,7 @@ static int attn_fused_plan(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64
     a.kv_heads = kv_heads, a.pos = pos, a.max_seq = max_seq, a.splits = splits, a.cps = cps;
     a.scratch_stride = stride;
     a.eps = eps, a.rope_base = rope_base, a.scale = scale;
+    a.spin_max = c->step_spin;
     if (splits > 1 || counters) {
         const int slot = sync_slot(c, s);
         if (slot < 0)
@@ -961,6 +964,11 @@ static int attn_fused_plan(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64
     return LP_OK;
 }
 
+// lp_attn_fused's workgroups: the splits, then (many splits) a merge per query head.
+static int attn_wgs(const AttnFusedArgs& a, int heads) {
+    return a.splits * a.kv_heads + (a.splits > kAttnLastMerge ? heads : 0);
+}
+
 int lp_attn_fused(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm, uint64_t k_norm, float eps,
                   float rope_base, uint64_t kcache, uint64_t vcache, uint64_t out, uint64_t scratch, int heads,
                   int kv_heads, int head_dim, int pos, int max_seq, float scale, lp_stream s) {
@@ -970,7 +978,7 @@ int lp_attn_fused(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm
     if (int r = attn_fused_plan(c, q, k, v, q_norm, k_norm, eps, rope_base, kcache, vcache, out, scratch, heads,
                                 kv_heads, head_dim, pos, max_seq, scale, false, s, a, gi))
         return r;
-    return launch(c, (Fn)(kAttnFusedG1 + gi), dim3((unsigned)a.splits, (unsigned)kv_heads), dim3(256), 0, s, a);
+    return launch(c, (Fn)(kAttnFusedG1 + gi), dim3((unsigned)attn_wgs(a, heads)), dim3(256), 0, s, a);
 }
 
 int lp_attn_block(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm, uint64_t k_norm, float eps,
@@ -991,8 +999,7 @@ int lp_attn_block(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm
         return r;
     b.wo = wo, b.h = h, b.ln = post_ln, b.hn = hn;
     b.rows = hidden, b.cols = cols;
-    b.n_attn = b.at.splits * kv_heads;
-    b.spin_max = c->step_spin;
+    b.n_attn = attn_wgs(b.at, heads);
     const unsigned n_o = (unsigned)((hidden + 4 * kBlockRowsPerWave - 1) / (4 * kBlockRowsPerWave));
     return launch(c, (Fn)(kAttnBlockG1 + gi), dim3((unsigned)b.n_attn + n_o), dim3(256), 0, s, b);
 }
