@@ -257,92 +257,119 @@ __device__ __forceinline__ uint32_t pack_i8x4(int a, int b, int c, int d) {
     return (uint32_t)(a & 255) | ((uint32_t)(b & 255) << 8) | ((uint32_t)(c & 255) << 16) | ((uint32_t)d << 24);
 }
 
-// One 32-column sub-group of an fp32 row as digits in operand order, its
-// seed -8 * sum xq and sigma.  p == 0 gives zeros (padding sub-groups,
-// missing tokens).
-struct DigitGroup {
-    uint4 hi[2], lo[2];
-    int32_t seed;
+// A sub-group by the four lanes of a quad: lane d (0..3) holds its columns 8 d
+// .. 8 d + 7 in v.  The largest magnitude and the sum of xq are shared by quad
+// permutations (exact: a maximum and an integer sum); the lane's eight columns'
+// digits are contiguous in operand order (even columns, then odd).  Whole
+// quads must call this together.  (One lane per sub-group read 128 bytes of
+// its own per 16-byte load, a cache line per lane, and converted 32 values in
+// a row: the one-token down + combine 8.4 us, 7.0 with quads.)
+struct QuadDigits {
+    uint2 hi, lo;
+    int32_t seed;  // -8 * sum xq
     float sigma;
 };
 
-__device__ __forceinline__ DigitGroup digit_group(const LP_GLOBAL float4* p) {
-    float v[32];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (p) f = p[i];
-        v[4 * i] = f.x;
-        v[4 * i + 1] = f.y;
-        v[4 * i + 2] = f.z;
-        v[4 * i + 3] = f.w;
-    }
+__device__ __forceinline__ QuadDigits quad_digits(const float (&v)[8]) {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) m = fmaxf(m, fabsf(v[i]));
-    DigitGroup q;
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));
+    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0xb1, 0xf, 0xf, false)));
+    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x4e, 0xf, 0xf, false)));
     const bool live = m >= kDigitMin;
     const float inv = live ? 32639.0f / m : 0.0f;
-    q.sigma = live ? m / 32639.0f : 0.0f;
-    int hi[32], lo[32], sum = 0;
+    int hi[8], lo[8], sum = 0;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) sum += digit_split(v[i], inv, hi[i], lo[i]);
+    for (int i = 0; i < 8; ++i) sum += digit_split(v[i], inv, hi[i], lo[i]);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xb1, 0xf, 0xf, false);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x4e, 0xf, 0xf, false);
+    QuadDigits q;
+    // columns 8d + {0, 2, 4, 6}, then 8d + {1, 3, 5, 7}
+    q.hi = make_uint2(pack_i8x4(hi[0], hi[2], hi[4], hi[6]), pack_i8x4(hi[1], hi[3], hi[5], hi[7]));
+    q.lo = make_uint2(pack_i8x4(lo[0], lo[2], lo[4], lo[6]), pack_i8x4(lo[1], lo[3], lo[5], lo[7]));
     q.seed = -8 * sum;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        uint32_t wh[4], wl[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int c0 = digit_col(h, 4 * w), c1 = digit_col(h, 4 * w + 1), c2 = digit_col(h, 4 * w + 2),
-                      c3 = digit_col(h, 4 * w + 3);
-            wh[w] = pack_i8x4(hi[c0], hi[c1], hi[c2], hi[c3]);
-            wl[w] = pack_i8x4(lo[c0], lo[c1], lo[c2], lo[c3]);
-        }
-        q.hi[h] = make_uint4(wh[0], wh[1], wh[2], wh[3]);
-        q.lo[h] = make_uint4(wl[0], wl[1], wl[2], wl[3]);
-    }
+    q.sigma = live ? m / 32639.0f : 0.0f;
     return q;
 }
 
-// Stage ntok activation rows into fragment pairs 0 .. ceil(ntok/2)-1.
-// row_of(t) returns the f32 row of token t.  Work units (token, sub-group)
-// are spread over the `nthreads` participating threads; a missing second
-// token of the last pair and the padding sub-groups are written as zeros.
-template <typename RowOf>
-__device__ inline void stage_rows(const Frags& F, int ntok, RowOf row_of, int tid, int nthreads) {
-    const int units = ((ntok + 1) & ~1) * F.ngp;
-    for (int u = tid; u < units; u += nthreads) {
-        const int t = u / F.ngp;
-        const int g = u - t * F.ngp;
-        const int pair = t >> 1, tk = t & 1;
-        const bool live = t < ntok && g < F.ng;
-        const DigitGroup q =
-            digit_group(live ? gptr<float4>(reinterpret_cast<uint64_t>(row_of(t) + (size_t)g * 32)) : nullptr);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            *reinterpret_cast<uint4*>(frag_ptr(F, pair, 2 * tk + 0, g) + h * 16) = q.hi[h];
-            *reinterpret_cast<uint4*>(frag_ptr(F, pair, 2 * tk + 1, g) + h * 16) = q.lo[h];
-        }
-        int32_t* of = off_ptr(F, pair, g);
-        of[2 * tk + 0] = 0;
-        of[2 * tk + 1] = q.seed;
-        sig_ptr(F, pair, g)[tk] = q.sigma;
-    }
+__device__ __forceinline__ void unpack8(const float4& a, const float4& b, float (&v)[8]) {
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-// Sub-group g of an fp32 row of `cols` columns into the row's digit image
-// (lpk::dimage_bytes layout).
-__device__ __forceinline__ void write_dimage_group(const float* row, int cols, int g, uint8_t* img) {
-    const int ng = cols >> 5, ngp = lpk::frag_ngp(cols);
-    const DigitGroup q =
-        digit_group(g < ng ? gptr<float4>(reinterpret_cast<uint64_t>(row + (size_t)g * 32)) : nullptr);
+// Stage ntok activation rows into fragment pairs 0 .. ceil(ntok/2)-1.
+// row_of(t) returns the f32 row of token t.  Work units (token, sub-group,
+// quarter) are spread over the `nthreads` (a multiple of 4) participating
+// threads, N units' loads in flight per thread; padding sub-groups are written as
+// zeros, the second token of an odd last pair is left as it is (its MFMA
+// output rows are separate and never stored).  between() is called once, when
+// the first units' loads have been issued and before they are waited for: the
+// caller's weight loads belong there, behind the rows in the memory queue
+// (loads land in order) and in flight during the conversion.
+template <int N = 2, typename RowOf, typename Between>
+__device__ __forceinline__ void stage_rows(const Frags& F, int ntok, RowOf row_of, int tid, int nthreads,
+                                           Between between) {
+    const int units = ntok * F.ngp * 4;
+    bool first = true;
+    for (int u0 = tid; first || u0 < units; u0 += N * nthreads) {
+        float4 f[N][2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        reinterpret_cast<uint4*>(img + (size_t)g * 32)[h] = q.hi[h];
-        reinterpret_cast<uint4*>(img + (size_t)ngp * 32 + (size_t)g * 32)[h] = q.lo[h];
+        for (int r = 0; r < N; ++r) {
+            const int gq = (u0 + r * nthreads) >> 2, t = gq / F.ngp, g = gq - t * F.ngp;
+            f[r][0] = f[r][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (t < ntok && g < F.ng) {
+                const LP_GLOBAL float4* p =
+                    gptr<float4>(reinterpret_cast<uint64_t>(row_of(t) + (size_t)g * 32)) + 2 * (u0 & 3);
+                f[r][0] = p[0];
+                f[r][1] = p[1];
+            }
+        }
+        if (first) between();
+        first = false;
+#pragma unroll
+        for (int r = 0; r < N; ++r) {
+            const int u = u0 + r * nthreads;
+            if (u >= units) break;
+            const int gq = u >> 2, t = gq / F.ngp, g = gq - t * F.ngp, d = u & 3;
+            const int pair = t >> 1, tk = t & 1;
+            float v[8];
+            unpack8(f[r][0], f[r][1], v);
+            const QuadDigits q = quad_digits(v);
+            *reinterpret_cast<uint2*>(frag_ptr(F, pair, 2 * tk + 0, g) + 8 * d) = q.hi;
+            *reinterpret_cast<uint2*>(frag_ptr(F, pair, 2 * tk + 1, g) + 8 * d) = q.lo;
+            if (d == 0) {
+                reinterpret_cast<int2*>(off_ptr(F, pair, g))[tk] = make_int2(0, q.seed);
+                sig_ptr(F, pair, g)[tk] = q.sigma;
+            }
+        }
     }
-    reinterpret_cast<int2*>(img + lpk::dimage_seed_off(ngp))[g] = make_int2(0, q.seed);
-    reinterpret_cast<float*>(img + lpk::dimage_sigma_off(ngp))[g] = q.sigma;
+}
+template <typename RowOf>
+__device__ inline void stage_rows(const Frags& F, int ntok, RowOf row_of, int tid, int nthreads) {
+    stage_rows(F, ntok, row_of, tid, nthreads, [] {});
+}
+
+// An fp32 row's digit image (lpk::dimage_bytes layout), by threads first,
+// first + step, ... of whole quads (step a multiple of 4).
+__device__ __forceinline__ void write_dimage(const float* row, int cols, uint8_t* img, int first, int step) {
+    const int ng = cols >> 5, ngp = lpk::frag_ngp(cols);
+    for (int u = first; u < 4 * ngp; u += step) {
+        const int g = u >> 2, d = u & 3;
+        float4 f0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), f1 = f0;
+        if (g < ng) {
+            f0 = *reinterpret_cast<const float4*>(row + g * 32 + d * 8);
+            f1 = *reinterpret_cast<const float4*>(row + g * 32 + d * 8 + 4);
+        }
+        float v[8];
+        unpack8(f0, f1, v);
+        const QuadDigits q = quad_digits(v);
+        *reinterpret_cast<uint2*>(img + (size_t)g * 32 + d * 8) = q.hi;
+        *reinterpret_cast<uint2*>(img + (size_t)ngp * 32 + (size_t)g * 32 + d * 8) = q.lo;
+        if (d == 0) {
+            reinterpret_cast<int2*>(img + lpk::dimage_seed_off(ngp))[g] = make_int2(0, q.seed);
+            reinterpret_cast<float*>(img + lpk::dimage_sigma_off(ngp))[g] = q.sigma;
+        }
+    }
 }
 
 // fp16 images (lpk::himage_bytes layout), the token operand of the prefill

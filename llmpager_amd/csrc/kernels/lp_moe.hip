@@ -60,66 +60,21 @@ __device__ __forceinline__ T load_agent(const LP_GLOBAL T* p) {
 // ---------------------------------------------------------------------------
 namespace {
 
-// Token t's digit image (the grouped kernels' A operand) from its row staged
-// in LDS, by the whole workgroup: the four threads of a sub-group take eight
-// columns each, share the sub-group's largest magnitude and their sum of xq
-// by quad permutations (exact: a maximum and an integer sum), and write their
-// eight columns' digits, which are contiguous in operand order (even columns,
-// then odd).  The same bytes as write_dimage_group.
-__device__ __forceinline__ void write_dimage_lds(const RouteArgs& a, int t, const float* row) {
-    const int H = a.L.hidden, ng = H >> 5, ngp = frag_ngp(H);
-    uint8_t* img = dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H);
-    for (int u = threadIdx.x; u < 4 * ngp; u += blockDim.x) {  // whole quads together
-        const int g = u >> 2, d = u & 3;
-        float v[8];
-        if (g < ng) {
-            const float4 f0 = *reinterpret_cast<const float4*>(row + g * 32 + d * 8);
-            const float4 f1 = *reinterpret_cast<const float4*>(row + g * 32 + d * 8 + 4);
-            v[0] = f0.x; v[1] = f0.y; v[2] = f0.z; v[3] = f0.w;
-            v[4] = f1.x; v[5] = f1.y; v[6] = f1.z; v[7] = f1.w;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-        }
-        float m = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));
-        m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0xb1, 0xf, 0xf, false)));
-        m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x4e, 0xf, 0xf, false)));
-        const bool live = m >= kDigitMin;
-        const float inv = live ? 32639.0f / m : 0.0f;
-        int hi[8], lo[8], sum = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sum += digit_split(v[i], inv, hi[i], lo[i]);
-        sum += __builtin_amdgcn_update_dpp(0, sum, 0xb1, 0xf, 0xf, false);
-        sum += __builtin_amdgcn_update_dpp(0, sum, 0x4e, 0xf, 0xf, false);
-        // columns 8d + {0, 2, 4, 6}, then 8d + {1, 3, 5, 7}
-        *reinterpret_cast<uint2*>(img + (size_t)g * 32 + d * 8) =
-            make_uint2(pack_i8x4(hi[0], hi[2], hi[4], hi[6]), pack_i8x4(hi[1], hi[3], hi[5], hi[7]));
-        *reinterpret_cast<uint2*>(img + (size_t)ngp * 32 + (size_t)g * 32 + d * 8) =
-            make_uint2(pack_i8x4(lo[0], lo[2], lo[4], lo[6]), pack_i8x4(lo[1], lo[3], lo[5], lo[7]));
-        if (d == 0) {
-            reinterpret_cast<int2*>(img + dimage_seed_off(ngp))[g] = make_int2(0, -8 * sum);
-            reinterpret_cast<float*>(img + dimage_sigma_off(ngp))[g] = live ? m / 32639.0f : 0.0f;
-        }
-    }
-}
-
 // Token t's images from its row in memory, by the whole workgroup.
 __device__ __forceinline__ void write_image(const RouteArgs& a, int t) {
     const int H = a.L.hidden;
     const float* row = dptr<const float>(a.x) + (size_t)t * H;
-    if (a.make_xf & kImgDigits) {
-        uint8_t* img = dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H);
-        for (int g = threadIdx.x; g < frag_ngp(H); g += blockDim.x) write_dimage_group(row, H, g, img);
-    }
+    if (a.make_xf & kImgDigits)
+        write_dimage(row, H, dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H), threadIdx.x, blockDim.x);
     if (a.make_xf & kImgF16)
         write_h16_image(row, H, dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(H), dptr<int>(a.W.xexp) + t);
 }
 
 // Token t's images from its row staged in LDS.
 __device__ __forceinline__ void write_images_lds(const RouteArgs& a, int t, const float* row) {
-    if (a.make_xf & kImgDigits) write_dimage_lds(a, t, row);
+    const int H = a.L.hidden;
+    if (a.make_xf & kImgDigits)
+        write_dimage(row, H, dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H), threadIdx.x, blockDim.x);
     if (a.make_xf & kImgF16)
         write_h16_image(row, a.L.hidden, dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(a.L.hidden),
                         dptr<int>(a.W.xexp) + t);
@@ -343,18 +298,16 @@ __device__ __forceinline__ void router_rows(const RouteArgs& a) {
 extern "C" __global__ void __launch_bounds__(256) lp_moe_router(const RouteArgs a) { router_rows(a); }
 
 // Images of x alone (callers that route from their own logits, and the
-// large-batch router): one wave per token, lane l converting sub-groups l,
-// l + 64, ... (digits) or 16-byte words l, l + 64, ... (fp16, after the row's
+// large-batch router): one wave per token, quads of lanes converting
+// sub-groups (digits) or 16-byte words l, l + 64, ... (fp16, after the row's
 // largest magnitude), and W.xexp[t].  Grid (ceil(T / 4)), 256 threads.
 extern "C" __global__ void __launch_bounds__(256) lp_moe_ximage(const RouteArgs a) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= a.T) return;
     const int H = a.L.hidden, lane = lane_id();
     const float* row = dptr<const float>(a.x) + (size_t)t * H;
-    if (a.make_xf & kImgDigits) {
-        uint8_t* img = dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H);
-        for (int g = lane; g < frag_ngp(H); g += 64) write_dimage_group(row, H, g, img);
-    }
+    if (a.make_xf & kImgDigits)
+        write_dimage(row, H, dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H), lane, 64);
     if (a.make_xf & kImgF16) {
         const int e = h16_exp(row_absmax_wave(row, H, lane, 64));
         uint8_t* img = dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(H);
@@ -1684,12 +1637,6 @@ __device__ __forceinline__ void down_bal_body(const GroupedArgs& a) {
         sblob[s] = P.x[s].blob;
         sp0[s] = P.x[s].p0 + tb;
         snt[s] = P.x[s].ntok - tb;
-        if (s < P.nslot) {
-            Frags Fs = F;
-            Fs.lds = F.lds + kBalGroups * kBalPairs * s * frag_pair_bytes(F.ngp);
-            const int p0 = sp0[s];
-            stage_rows(Fs, P.ns[s], [&](int t) { return actp + (size_t)(p0 + t) * I; }, threadIdx.x, blockDim.x);
-        }
     }
     // this wave's units: lo + wave + W * j < hi
     const int J = hi - lo > wave ? (hi - lo - wave + W - 1) / W : 0;
@@ -1759,8 +1706,19 @@ __device__ __forceinline__ void down_bal_body(const GroupedArgs& a) {
             }
         }
     };
+    // the slots' act rows, the first unit's weights behind the first of them
     WRegs<NS, SL> RA[TW];
-    load(RA, 0, swin);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        if (s < P.nslot) {
+            Frags Fs = F;
+            Fs.lds = F.lds + kBalGroups * kBalPairs * s * frag_pair_bytes(F.ngp);
+            const int p0 = sp0[s];
+            stage_rows(Fs, P.ns[s], [&](int t) { return actp + (size_t)(p0 + t) * I; }, threadIdx.x, blockDim.x, [&] {
+                if (s == 0) load(RA, 0, swin);
+            });
+        }
+    }
     __builtin_amdgcn_s_waitcnt(0);  // the first unit has landed
     __syncthreads();                // and the staged act rows are in place
     for (int j = 0; j < J; ++j) {
@@ -1821,19 +1779,35 @@ __device__ __forceinline__ void down_group(const Frags& F, WRegs<NS, SL> (&D)[TW
     }
 }
 
+// The matrices and tables one workgroup of the one-shot down works on: the
+// routed experts', or (lp_moe_down_wide's workgroups from sh_wg0 on) the
+// shared MLP's.
+struct DownView {
+    uint64_t et, act, y, down_off;
+    int inter, group, wg;  // wg: the workgroup's index among its own kind
+    bool routed;
+};
+
+__device__ __forceinline__ DownView down_view(const GroupedArgs& a) {
+    const int b = (int)blockIdx.x;
+    if (a.sh_wg0 > 0 && b >= a.sh_wg0)
+        return DownView{a.W.sh_et, a.W.sh_act, a.W.sh_y, a.L.sh_down_off, a.L.shared_inter, a.L.shared_group,
+                        b - a.sh_wg0, false};
+    return DownView{a.W.et, a.W.act, a.W.y, a.L.down_off, a.L.inter, a.L.group, b, true};
+}
+
 template <int TW, int NS, bool ONE, int RS, bool SL>
-__device__ __forceinline__ void down_body(const GroupedArgs& a) {
+__device__ __forceinline__ void down_body(const GroupedArgs& a, const DownView& V) {
     extern __shared__ __align__(16) uint8_t lds[];
-    const LayerView& L = a.L;
-    const int H = L.hidden, I = L.inter;
+    const int H = a.L.hidden, I = V.inter;
     const int wave = threadIdx.x >> 6, W = blockDim.x >> 6;
     const int run = kTileRows * W * TW;
     const int chunks = (H + run - 1) / run;
-    const int u = blockIdx.x / chunks;
-    const int chunk = blockIdx.x - u * chunks;
-    const ExpertEntry x = entry_of(a, u);
+    const int u = V.wg / chunks;
+    const int chunk = V.wg - u * chunks;
+    const ExpertEntry x = entry_at(V.et, u);
     if (x.ntok == 0) return;
-    float* y = dptr<float>(a.W.y);
+    float* y = dptr<float>(V.y);
     if (x.blob == 0) {
         missing_expert(a, x, y, H, H, chunk * run, chunk * run + run);
         return;
@@ -1849,18 +1823,20 @@ __device__ __forceinline__ void down_body(const GroupedArgs& a) {
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
         n0[t] = chunk * run + kTileRows * (wave + W * t);
-        TD[t] = wtile<RS>(x.blob + L.down_off, H, I, n0[t]);
-        wload(D[t], TD[t], 0, swin + (uint32_t)(t * scale_window_bytes<NS>()));
+        TD[t] = wtile<RS>(x.blob + V.down_off, H, I, n0[t]);
     }
     zero_block(F, threadIdx.x, blockDim.x);
-    const float* act = dptr<const float>(a.W.act);
+    const float* act = dptr<const float>(V.act);
     const int cap = min(kMaxPairs, a.pairs_cap);
     for (int tb = 0; tb < x.ntok; tb += 2 * cap) {
         const int nt = min(2 * cap, x.ntok - tb);
         const bool reload = tb + nt < x.ntok;
         if (tb > 0) __syncthreads();
-        stage_rows(F, nt, [&](int t) { return act + (size_t)(x.p0 + tb + t) * I; },
-                   threadIdx.x, blockDim.x);
+        stage_rows<TW == 1 ? 4 : 2>(F, nt, [&](int t) { return act + (size_t)(x.p0 + tb + t) * I; }, threadIdx.x, blockDim.x, [&] {
+            if (tb > 0) return;
+#pragma unroll
+            for (int t = 0; t < TW; ++t) wload(D[t], TD[t], 0, swin + (uint32_t)(t * scale_window_bytes<NS>()));
+        });
         __syncthreads();
         down_group<kMaxPairs, TW, NS, ONE, RS, SL>(F, D, TD, H, n0, S, tb, nt, x.p0, reload, y);
     }
@@ -1952,43 +1928,49 @@ lp_moe_down_bal6(const GroupedArgs a) {
 // picks this kernel only for those), loaded in one piece.
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lp_moe_down(const GroupedArgs a) {
-    if (scales_in_lds(a.L.group, a.L.inter)) {
+    const DownView V = down_view(a);
+    if (scales_in_lds(V.group, V.inter)) {
         // a 6-step tile (inter 768) loads only its own 6 steps
-        if (tile_steps(a.L.inter) == 6)
-            down_body<2, 6, true, 0, true>(a);
+        if (tile_steps(V.inter) == 6)
+            down_body<2, 6, true, 0, true>(a, V);
         else
-            down_body<2, kDownChunk, true, 0, true>(a);
+            down_body<2, kDownChunk, true, 0, true>(a, V);
     } else {
-#define LP_DOWN(rs) down_body<2, kDownChunk, true, rs, false>(a)
-        LP_BY_RS(a.L.group, LP_DOWN)
+#define LP_DOWN(rs) down_body<2, kDownChunk, true, rs, false>(a, V)
+        LP_BY_RS(V.group, LP_DOWN)
 #undef LP_DOWN
     }
 }
 
 // Down, one row tile per wave: up to kDownWideChunk steps in one piece,
-// longer tiles streamed kDownLoopChunk steps at a time.
+// longer tiles streamed kDownLoopChunk steps at a time.  Workgroups from
+// sh_wg0 on take the shared MLP's entries (its own width and group): both
+// downs of a DeepSeek-V2-Lite-shape layer of 16 tokens in one launch 31.1
+// us, 18.3 + 18.3 in two (the shared one's few workgroups leave the chip
+// idle on their own).
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lp_moe_down_wide(const GroupedArgs a) {
-    const int S = tile_steps(a.L.inter);
+    const DownView V = down_view(a);
+    const int S = tile_steps(V.inter);
     if (S <= kDownWideChunk) {
         // tiles of 9..12 steps (inter 1152..1536) load 12 steps, not 16
-        if (scales_in_lds(a.L.group, a.L.inter)) {
+        if (scales_in_lds(V.group, V.inter)) {
             if (S <= 12)
-                down_body<1, 12, true, 0, true>(a);
+                down_body<1, 12, true, 0, true>(a, V);
             else
-                down_body<1, kDownWideChunk, true, 0, true>(a);
+                down_body<1, kDownWideChunk, true, 0, true>(a, V);
         } else if (S <= 12) {
-#define LP_DOWN(rs) down_body<1, 12, true, rs, false>(a)
-            LP_BY_RS(a.L.group, LP_DOWN)
+#define LP_DOWN(rs) down_body<1, 12, true, rs, false>(a, V)
+            LP_BY_RS(V.group, LP_DOWN)
 #undef LP_DOWN
         } else {
-#define LP_DOWN(rs) down_body<1, kDownWideChunk, true, rs, false>(a)
-            LP_BY_RS(a.L.group, LP_DOWN)
+#define LP_DOWN(rs) down_body<1, kDownWideChunk, true, rs, false>(a, V)
+            LP_BY_RS(V.group, LP_DOWN)
 #undef LP_DOWN
         }
     } else {
-#define LP_DOWN(rs) down_body<1, kDownLoopChunk, false, rs, false>(a)
-        LP_BY_RS(a.L.group, LP_DOWN)
+#define LP_DOWN(rs) down_body<1, kDownLoopChunk, false, rs, false>(a, V)
+        LP_BY_RS(V.group, LP_DOWN)
 #undef LP_DOWN
     }
 }
@@ -2146,17 +2128,16 @@ __device__ __forceinline__ void down_comb_body(const GroupedArgs& a) {
     WRegs<NS, SL> D;
     if (blob != 0) {
         const WTile<RS> T = wtile<RS>(blob + L.down_off, H, I, n0);
-        wload(D, T, 0, swin);
         Frags Fw = F;
         Fw.lds = F.lds + wave * frag_pair_bytes(F.ngp);
         const float* actp = dptr<const float>(a.W.act);
-        stage_rows(Fw, 1, [&](int) { return actp + (size_t)p * I; }, lane, 64);
+        stage_rows<NS == 16 ? 4 : 2>(Fw, 1, [&](int) { return actp + (size_t)p * I; }, lane, 64,
+                                     [&] { wload(D, T, 0, swin); });
     } else if (shw) {
         const WTile<RS> T = wtile<RS>(L.shared_blob + L.sh_down_off, H, Is, n0);
-        wload(D, T, q * hs, swin);
         const float* sact = dptr<const float>(a.W.sh_act);
         stage_rows(Fs, 1, [&](int) { return sact; }, (int)threadIdx.x - 64 * (kCombWaves - kCombShWaves),
-                   64 * kCombShWaves);
+                   64 * kCombShWaves, [&] { wload(D, T, q * hs, swin); });
     }
     __builtin_amdgcn_s_waitcnt(0);  // the tile, its scale window and the staged row
     __syncthreads();

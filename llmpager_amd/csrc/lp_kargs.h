@@ -391,7 +391,7 @@ struct GroupedArgs {
     int32_t sh_maxu;     // balanced gate/up: the shared MLP's W.sh_et entries taken after the routed ones
     int32_t wave_u0;     // combine of one wave (wave_n > 0): the routed experts uniq[wave_u0 ..
     int32_t wave_n;      //   wave_u0 + wave_n) only; tokens without a pick among them are left as they are
-    int32_t pad0;
+    int32_t sh_wg0;      // lp_moe_down_wide: the first workgroup of the shared MLP's down (0: routed only)
 };
 
 // Balanced decode gate/up (lp_moe_gateup_bal): one workgroup of kBalWaves

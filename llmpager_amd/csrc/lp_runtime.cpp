@@ -1352,11 +1352,16 @@ static bool down_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
 }
 
 // The grouped down projection of ga's entries (maxu): balanced for routed
-// decode batches when it can, else the one-shot kernels.
-static int grouped_down(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed, lp_stream s) {
+// decode batches when it can, else the one-shot kernels.  sh_entries > 0
+// (routed only): where that is lp_moe_down_wide, the shared MLP's entries
+// (its gate/up already done) in the same launch; *sh_done says whether.
+static int grouped_down(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed, lp_stream s, int sh_entries = 0,
+                        bool* sh_done = nullptr) {
     GroupedArgs ga = ga0;
     ga.maxu = maxu;
     ga.sh_maxu = 0;
+    ga.sh_wg0 = 0;
+    if (sh_done) *sh_done = false;
     const int H = ga.L.hidden, I = ga.L.inter, cap = ga.pairs_cap;
     // Waves per workgroup: the most that still give every CU two workgroups
     // (routed) or one (the shared MLP: its few entries' act rows, staged by
@@ -1379,9 +1384,20 @@ static int grouped_down(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed
     const int w = pick_w(H, tw);
     const int chunks = (H + kTileRows * w * tw - 1) / (kTileRows * w * tw);
     const int ns = steps <= kDownChunk ? kDownChunk : kDownWideChunk;
-    const int win = steps <= kDownWideChunk && scales_in_lds(ga.L.group, I) ? scale_window_lds(w, tw, ns) : 0;
-    return launch(c, f, dim3((unsigned)(maxu * chunks)), dim3(64 * w), (size_t)(frag_lds_bytes(I, cap) + win),
-                  s, ga);
+    auto lds_of = [&](int inter, int group) {
+        const int win = tile_steps_host(inter) <= kDownWideChunk && scales_in_lds(group, inter)
+                            ? scale_window_lds(w, tw, ns) : 0;
+        return (size_t)(frag_lds_bytes(inter, cap) + win);
+    };
+    size_t lds = lds_of(I, ga.L.group);
+    unsigned wgs = (unsigned)(maxu * chunks);
+    if (sh_entries > 0 && f == kDownWide) {
+        ga.sh_wg0 = (int)wgs;
+        wgs += (unsigned)(sh_entries * chunks);
+        lds = std::max(lds, lds_of(ga.L.shared_inter, ga.L.shared_group));
+        *sh_done = true;
+    }
+    return launch(c, f, dim3(wgs), dim3(64 * w), lds, s, ga);
 }
 
 // Grouped gate/up (+ SiLU) and down over the work items of ga's expert table
@@ -1392,13 +1408,15 @@ static int grouped_down(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed
 // entries of one blob, whose weight rows neighbouring workgroups of one XCD
 // read together).
 // sh_maxu > 0 (routed only): the balanced gate/up also takes the shared
-// MLP's entries when it can; *sh_done says whether it did.
+// MLP's entries when it can; *sh_done says whether it did, *sh_down whether
+// the down did too.
 static int grouped_ffn(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed, lp_stream s,
-                       bool with_down = true, int sh_maxu = 0, bool* sh_done = nullptr) {
+                       bool with_down = true, int sh_maxu = 0, bool* sh_done = nullptr, bool* sh_down = nullptr) {
     GroupedArgs ga = ga0;
     ga.maxu = maxu;
     ga.sh_maxu = 0;
     if (sh_done) *sh_done = false;
+    if (sh_down) *sh_down = false;
     // (the 16-step form with scales in LDS windows only: its own kernel)
     if (sh_maxu > 0 && c->gateup_bal && tile_steps_host(ga.L.hidden) > 8 && scales_in_lds(ga.L.group, ga.L.hidden)) {
         GroupedArgs gs = ga;
@@ -1433,7 +1451,9 @@ static int grouped_ffn(lp_ctx* c, const GroupedArgs& ga0, int maxu, bool routed,
             return r;
     }
     if (!with_down) return 0;
-    return grouped_down(c, ga0, maxu, routed, s);
+    // the shared MLP's down may ride along once its gate/up has
+    const bool ride = sh_down && sh_done && *sh_done;
+    return grouped_down(c, ga0, maxu, routed, s, ride ? sh_maxu : 0, sh_down);
 }
 
 // LDS of lp_moe_down_comb(16, _rs): the picks' fragment pairs, their row
@@ -1568,7 +1588,7 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
     if (lds_for(1) > c->max_lds)
         return fail(LP_E_UNSUPPORTED, "hidden/inter too large for one LDS fragment pair");
     ga.pairs_cap = cap;
-    bool sh_gu = false;  // the shared MLP's gate/up done by the routed launch
+    bool sh_gu = false, sh_dn = false;  // the shared MLP's gate/up, its down done by the routed launches
     if (!wave && use_gemm(d, T)) {
         if ((size_t)kGemmLds > c->max_lds) return fail(LP_E_UNSUPPORTED, "GEMM stages exceed the LDS");
         // the GEMM loads address images and weights as 32-bit offsets from a base
@@ -1606,7 +1626,7 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         // the groups agree (sh_gu: it did)
         const int shm =
             !wave && d->shared_blob && d->shared_group == d->group && !use_mid_shared(d, T) ? shared_entries(T) : 0;
-        if (int r = grouped_ffn(c, ga, maxu, true, s, !comb, shm, &sh_gu)) return r;
+        if (int r = grouped_ffn(c, ga, maxu, true, s, !comb, shm, &sh_gu, &sh_dn)) return r;
         if (comb) {
             const Fn f = !sl ? kDownCombRs : Si <= 8 ? kDownComb : kDownComb16;
             // the shared MLP's down on the comb kernel's idle waves: per-lane
@@ -1627,7 +1647,7 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
     }
     if (use_mid_shared(d, T)) {
         if (int r = mid_shared_ffn(c, d, ga, T, s)) return r;
-    } else if (d->shared_blob) {
+    } else if (d->shared_blob && !sh_dn) {
         if (int r = shared_ffn(c, d, ga, T, s, true, !sh_gu)) return r;
     }
     return launch(c, kCombine, dim3((unsigned)((d->hidden + 1023) / 1024), (unsigned)T), dim3(256), 0,
