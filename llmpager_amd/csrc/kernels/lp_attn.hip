@@ -53,17 +53,60 @@ __device__ __forceinline__ uint16_t f32_to_half_bits(float f) {
 
 // ---------------------------------------------------------------------------
 // RMSNorm per row (decode.cu:17-41): y[r] = x[r] * 1/sqrt(mean(x[r]^2) + eps)
-// * w.  One workgroup of 256 per row; w is shared by all rows; y may be x.
+// * w; w is shared by all rows; y may be x.  Rows of up to 1024 elements take
+// a wave each (four per workgroup, no barrier), longer ones a workgroup; a
+// row whose pieces are 16-byte aligned and at most 4 per thread is read once,
+// with w, in one round of loads and kept in registers.  (One workgroup per
+// row whatever its width, element by element and twice: 5.1 us on average
+// over a decode layer's 1 x 2048, 32 x 128 and 4 x 128 norms, 2.6 now.)
 // ---------------------------------------------------------------------------
 extern "C" __global__ void __launch_bounds__(256) lp_rmsnorm(const RmsNormArgs a) {
     __shared__ float red[4];
-    const float* x = dptr<const float>(a.x) + (size_t)blockIdx.x * a.n;
-    float* y = dptr<float>(a.y) + (size_t)blockIdx.x * a.n;
+    const int per = a.wave_rows ? 64 : 256, i0 = a.wave_rows ? lane_id() : (int)threadIdx.x;
+    const int row = a.wave_rows ? (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6) : (int)blockIdx.x;
+    if (row >= a.rows) return;  // whole waves; with a workgroup per row, none
+    const uint64_t xp = a.x + (uint64_t)row * (uint32_t)a.n * 4u, yp = a.y + (uint64_t)row * (uint32_t)a.n * 4u;
+    auto total = [&](float v) {
+        if (!a.wave_rows) return block_sum(v, red);
+        for (int o = 32; o >= 1; o >>= 1) v += shfl_xor(v, o);
+        return v;
+    };
+    if ((a.n & 3) == 0 && ((xp | yp | a.w) & 15) == 0 && a.n <= 16 * per) {
+        float4 x[4], w[4];
+        float acc = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j * per;
+            x[j] = w[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (4 * i < a.n) {
+                x[j] = gptr<float4>(xp)[i];
+                w[j] = gptr<float4>(a.w)[i];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            acc = __builtin_fmaf(x[j].x, x[j].x, acc);
+            acc = __builtin_fmaf(x[j].y, x[j].y, acc);
+            acc = __builtin_fmaf(x[j].z, x[j].z, acc);
+            acc = __builtin_fmaf(x[j].w, x[j].w, acc);
+        }
+        const float inv = 1.0f / sqrtf(total(acc) / (float)a.n + a.eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j * per;
+            if (4 * i < a.n)
+                gptr_w<float4>(yp)[i] = make_float4(x[j].x * inv * w[j].x, x[j].y * inv * w[j].y,
+                                                    x[j].z * inv * w[j].z, x[j].w * inv * w[j].w);
+        }
+        return;
+    }
+    const float* x = dptr<const float>(xp);
     const float* w = dptr<const float>(a.w);
+    float* y = dptr<float>(yp);
     float acc = 0.0f;
-    for (int i = threadIdx.x; i < a.n; i += 256) acc = __builtin_fmaf(x[i], x[i], acc);
-    const float inv = 1.0f / sqrtf(block_sum(acc, red) / (float)a.n + a.eps);
-    for (int i = threadIdx.x; i < a.n; i += 256) y[i] = x[i] * inv * w[i];
+    for (int i = i0; i < a.n; i += per) acc = __builtin_fmaf(x[i], x[i], acc);
+    const float inv = 1.0f / sqrtf(total(acc) / (float)a.n + a.eps);
+    for (int i = i0; i < a.n; i += per) y[i] = x[i] * inv * w[i];
 }
 
 // a += s * b (decode.cu:44-53)

@@ -15,31 +15,45 @@ using namespace lpk;
 // Requires group = 32 * 2^r, 16-byte aligned nibble rows and x (host checks).
 // Dynamic LDS: lpk::frag_lds_bytes(cols, 1).
 // ---------------------------------------------------------------------------
-template <int RS>
-__device__ __forceinline__ void q4_gemv_tiles(const Q4GemvBatchArgs& a, const Frags& F, uint64_t region,
+// One workgroup: the wave's first tile's first chunk (up to kGemvChunk steps,
+// or all of a tile of up to 2 kGemvChunk: ONE) is loaded behind x's row and
+// stays in flight while the row is converted.
+template <int NS, bool ONE, int RS>
+__device__ __forceinline__ void q4_gemv_tiles(const Q4GemvBatchArgs& a, const Frags& F, uint64_t region, const float* x,
                                               float* y) {
     const int wave = threadIdx.x >> 6;
     const int wpb = blockDim.x >> 6;
     const int lane = lane_id();
     const int tiles = (a.rows + kTileRows - 1) / kTileRows;
     const int S = tile_steps(a.cols);
-    for (int tile = blockIdx.x * wpb + wave; tile < tiles; tile += gridDim.x * wpb) {
-        const int n0 = tile * kTileRows;
-        const WTile<RS> T = wtile<RS>(region, a.rows, a.cols, n0);
+    int tile = blockIdx.x * wpb + wave;
+    WTile<RS> T = wtile<RS>(region, a.rows, a.cols, kTileRows * min(tile, tiles - 1));
+    WRegs<NS> R[1];
+    zero_block(F, threadIdx.x, blockDim.x);
+    stage_rows<4>(F, 1, [&](int) { return x; }, threadIdx.x, blockDim.x, [&] { wload(R[0], T, 0); });
+    __syncthreads();
+    for (; tile < tiles; tile += gridDim.x * wpb) {
         float acc[1][1][2] = {{{0.0f, 0.0f}}};
-        WRegs<kGemvChunk> R[1];
-        wload(R[0], T, 0);
+        if constexpr (ONE) {
+            const ABase B[1] = {abase(F, 0, 0)};
+            wmma(R, B, S, 1, acc);
+        } else {
 #pragma nounroll
-        for (int c0 = 0;;) {
-            const ABase B[1] = {abase(F, 0, c0)};
-            wmma(R, B, S - c0, 1, acc);
-            c0 += kGemvChunk;
-            if (c0 >= S) break;
-            wload(R[0], T, c0);
+            for (int c0 = 0;;) {
+                const ABase B[1] = {abase(F, 0, c0)};
+                wmma(R, B, S - c0, 1, acc);
+                c0 += NS;
+                if (c0 >= S) break;
+                wload(R[0], T, c0);
+            }
         }
         const float v = tile_reduce(acc[0][0][0]);
-        const int row = n0 + (lane & 15);
+        const int row = kTileRows * tile + (lane & 15);
         if (lane < 16 && row < a.rows) y[row] = v;
+        if (tile + gridDim.x * wpb < tiles) {
+            T = wtile<RS>(region, a.rows, a.cols, kTileRows * (tile + gridDim.x * wpb));
+            wload(R[0], T, 0);
+        }
     }
 }
 
@@ -50,14 +64,20 @@ extern "C" __global__ void __launch_bounds__(256) lp_q4_gemv_mfma(const Q4GemvBa
     const float* x = reinterpret_cast<const float*>(a.x) + (size_t)e * a.x_stride;
     float* y = reinterpret_cast<float*>(a.y) + (size_t)e * a.rows;
     const Frags F = frags_at(lds, a.cols);
-    zero_block(F, threadIdx.x, blockDim.x);
-    stage_rows(F, 1, [&](int) { return x; }, threadIdx.x, blockDim.x);
-    __syncthreads();
+    const int S = tile_steps(a.cols);
+#define LP_GEMV(rs)                                                                        \
+    if (S <= kGemvChunk)                                                                   \
+        q4_gemv_tiles<kGemvChunk, true, rs>(a, F, region, x, y);                           \
+    else if (S <= 2 * kGemvChunk)                                                          \
+        q4_gemv_tiles<2 * kGemvChunk, true, rs>(a, F, region, x, y);                       \
+    else                                                                                   \
+        q4_gemv_tiles<kGemvChunk, false, rs>(a, F, region, x, y);
     switch (ilog2_pow2(a.group >> 5)) {
-        case 0: q4_gemv_tiles<0>(a, F, region, y); break;
-        case 1: q4_gemv_tiles<1>(a, F, region, y); break;
-        default: q4_gemv_tiles<2>(a, F, region, y); break;
+        case 0: LP_GEMV(0) break;
+        case 1: LP_GEMV(1) break;
+        default: LP_GEMV(2) break;
     }
+#undef LP_GEMV
 }
 
 // Generic VALU form for any group % 8 == 0 (and unaligned operands): one wave
@@ -97,9 +117,21 @@ extern "C" __global__ void __launch_bounds__(256) lp_moe_reduce(const MoeReduceA
     const float* w = reinterpret_cast<const float*>(a.wts);
     float* out = reinterpret_cast<float*>(a.out);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+        const float o = out[i];
         float acc = 0.0f;
-        for (int e = 0; e < a.experts; ++e) acc = __builtin_fmaf(w[e], eo[(size_t)e * a.n + i], acc);
-        out[i] += acc;
+        for (int e0 = 0; e0 < a.experts; e0 += 8) {  // eight experts' loads in flight
+            float v[8], wt[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int e = min(e0 + j, a.experts - 1);
+                v[j] = eo[(size_t)e * a.n + i];
+                wt[j] = w[e];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (e0 + j < a.experts) acc = __builtin_fmaf(wt[j], v[j], acc);
+        }
+        out[i] = o + acc;
     }
 }
 
@@ -136,10 +168,8 @@ extern "C" __global__ void __launch_bounds__(256) lp_bf16_gemv(const Bf16GemvArg
     const int chunks = a.cols >> 3;
     const bool vec = (a.cols & 7) == 0;
     if (vec) {
-        for (int ch = lane; ch < chunks; ch += 64) {
-            const uint4 wv = *reinterpret_cast<const uint4*>(w + ch * 8);
-            const float4 xa = *reinterpret_cast<const float4*>(x + ch * 8);
-            const float4 xb = *reinterpret_cast<const float4*>(x + ch * 8 + 4);
+        const uint64_t wp = reinterpret_cast<uint64_t>(w), xp = a.x;
+        auto add = [&](const uint4& wv, const float4& xa, const float4& xb) {
             acc = __builtin_fmaf(bf16_to_f32(wv.x & 0xffffu), xa.x, acc);
             acc = __builtin_fmaf(bf16_to_f32(wv.x >> 16), xa.y, acc);
             acc = __builtin_fmaf(bf16_to_f32(wv.y & 0xffffu), xa.z, acc);
@@ -148,7 +178,25 @@ extern "C" __global__ void __launch_bounds__(256) lp_bf16_gemv(const Bf16GemvArg
             acc = __builtin_fmaf(bf16_to_f32(wv.z >> 16), xb.y, acc);
             acc = __builtin_fmaf(bf16_to_f32(wv.w & 0xffffu), xb.z, acc);
             acc = __builtin_fmaf(bf16_to_f32(wv.w >> 16), xb.w, acc);
+        };
+        // four chunks' loads in flight, the row's (from memory) first
+        int c0 = 0;
+        for (; c0 + 256 <= chunks; c0 += 256) {
+            uint4 wv[4];
+            float4 xa[4], xb[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) wv[j] = gptr<uint4>(wp)[c0 + 64 * j + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                xa[j] = gptr<float4>(xp)[2 * (c0 + 64 * j + lane)];
+                xb[j] = gptr<float4>(xp)[2 * (c0 + 64 * j + lane) + 1];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) add(wv[j], xa[j], xb[j]);
         }
+        for (int ch = c0 + lane; ch < chunks; ch += 64)
+            add(gptr<uint4>(wp)[ch], gptr<float4>(xp)[2 * ch], gptr<float4>(xp)[2 * ch + 1]);
     } else {
         for (int c = lane; c < a.cols; c += 64) acc = __builtin_fmaf(bf16_to_f32(w[c]), x[c], acc);
     }

@@ -187,10 +187,12 @@ struct ExpfSweepArgs {              // device expf check (no reference counterpa
 
 // ---- the rest of the decode step (decode.cu) and MLA (mla.cu) ----------------
 
-struct RmsNormArgs {                // kernels.rs:145-158 (rmsnorm_f32); rows = grid
+struct RmsNormArgs {                // kernels.rs:145-158 (rmsnorm_f32)
     uint64_t x, w, y;
     int32_t n;
     float eps;
+    int32_t rows;
+    int32_t wave_rows;              // a wave per row, four rows per workgroup (else a workgroup per row)
 };
 
 struct ScaleAddArgs {               // kernels.rs:161-173 (scale_add_f32)

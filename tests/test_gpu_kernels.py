@@ -128,3 +128,64 @@ def test_device_expf_matches_glibc(cuda, first, stride, n):
     want = O.expf_sweep(first, stride, n)
     same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
     assert same.all(), hex((first + stride * int(np.argmin(same))) & 0xffffffff)
+
+
+# The 1:1 launchers' edges: rows around a wave's and a workgroup's register
+# form of rmsnorm, widths that make no 16-byte pieces; bf16 GEMV widths around
+# four chunks of 64 lanes; q4 GEMV tiles of one chunk, of two and of more, on
+# one wave per workgroup and on four.  Bounds: fp32 sums of n terms.
+@pytest.mark.parametrize("rows,n", [(1, 1024), (5, 1023), (3, 1028), (2, 4096), (2, 4100), (7, 20), (9, 30)])
+def test_rmsnorm_edges(cuda, rows, n):
+    rng = np.random.default_rng(n)
+    K = lp.Kernels(cuda)
+    x, w = rng.standard_normal(rows * n).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    dx, dw = cuda.upload(x), cuda.upload(w)
+    K.rmsnorm(dx, dw, dx, rows, n, 1e-6)
+    x64 = x.reshape(rows, n).astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6) * w
+    got = cuda.download(dx, (rows, n), np.float32)
+    assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1.0)) <= n * 2.0 ** -24 + 4 * 2.0 ** -23
+    cuda.free_device(dx)
+    cuda.free_device(dw)
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 8), (4, 2040), (3, 2048), (6, 2056), (2, 4096), (1, 4104), (3, 12288), (4, 2047)])
+def test_bf16_gemv_edges(cuda, rows, cols):
+    K = lp.Kernels(cuda)
+    w = lp.synth_bf16(rows * cols, 0.05, 3, cols)
+    x = np.random.default_rng(cols).standard_normal(cols).astype(np.float32)
+    dw, dx, dy = cuda.upload(w), cuda.upload(x), cuda.alloc_device(rows * 4)
+    K.bf16_gemv(dw, dx, dy, rows, cols)
+    w64 = (w.astype(np.uint32) << 16).view(np.float32).astype(np.float64).reshape(rows, cols)
+    got = cuda.download(dy, (rows,), np.float32)
+    bound = (cols / 64 + 8) * 2.0 ** -24 * (np.abs(w64) @ np.abs(x.astype(np.float64)))
+    assert np.all(np.abs(got - w64 @ x) <= bound)
+    for p in (dw, dx, dy):
+        cuda.free_device(p)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("rows,cols,experts", [(16, 128, 1), (33, 1024, 2), (768, 1152, 8), (48, 2048, 3), (64, 2176, 2),
+                                               (2048, 768, 8), (5000, 256, 4)])
+def test_q4_gemv_batch_edges(cuda, rows, cols, experts, group):
+    rng = np.random.default_rng(rows + cols)
+    K = lp.Kernels(cuda)
+    gpr = cols // group
+    s = (rng.random((experts, rows, gpr)) * 0.05).astype(np.float16)
+    nib = rng.integers(0, 256, (experts, rows, cols // 2), dtype=np.uint8)
+    blobs = [np.concatenate([s[e].view(np.uint8).ravel(), nib[e].ravel()]) for e in range(experts)]
+    dev = [cuda.upload(b) for b in blobs]
+    dptr = cuda.upload(np.array([int(d) for d in dev], np.uint64))
+    x = rng.standard_normal((experts, cols)).astype(np.float32)
+    dx, dy = cuda.upload(x), cuda.alloc_device(experts * rows * 4)
+    K.q4g64_gemv_batch(dptr, 0, dx, cols, dy, rows, cols, group, experts)
+    q = np.stack([nib & 15, nib >> 4], -1).reshape(experts, rows, gpr, group).astype(np.float64) - 8
+    W = (q * s.astype(np.float64)[..., None]).reshape(experts, rows, cols)
+    got = cuda.download(dy, (experts, rows), np.float32)
+    for e in range(experts):
+        want = W[e] @ x[e].astype(np.float64)
+        # x to 2^-16 of each 32 columns' largest (at most max |x|), and fp32 sums
+        bound = (2.0 ** -16 * np.abs(x[e]).max() + 2.0 ** -24 * cols / 32 * np.abs(x[e]).max()) * np.abs(W[e]).sum(1)
+        assert np.all(np.abs(got[e] - want) <= bound)
+    for p in dev + [dptr, dx, dy]:
+        cuda.free_device(p)
