@@ -239,4 +239,3 @@ def test_mla_attn_decode_edges(cuda, K, heads, qk, cd, seq, ms):
     want = O.mla_attn_decode(q, cache[:seq * qk], heads, qk, cd, seq, scale)
     assert worst_rel(cuda.download(dctx, (heads * cd,), np.float32), want) <= 2.0 * np.sqrt(qk) * qk * 2.0 ** -24
     _free(cuda, dq, dc, dctx, dscr)
-

@@ -170,17 +170,14 @@ def test_bf16_gemv_edges(cuda, rows, cols):
 def test_q4_gemv_batch_edges(cuda, rows, cols, experts, group):
     rng = np.random.default_rng(rows + cols)
     K = lp.Kernels(cuda)
-    gpr = cols // group
-    s = (rng.random((experts, rows, gpr)) * 0.05).astype(np.float16)
-    nib = rng.integers(0, 256, (experts, rows, cols // 2), dtype=np.uint8)
-    blobs = [np.concatenate([s[e].view(np.uint8).ravel(), nib[e].ravel()]) for e in range(experts)]
+    w = rng.standard_normal((experts, rows * cols)).astype(np.float32) * 0.05
+    blobs = [O.q4_quantize(w[e], rows, cols, group)[0] for e in range(experts)]
     dev = [cuda.upload(b) for b in blobs]
     dptr = cuda.upload(np.array([int(d) for d in dev], np.uint64))
     x = rng.standard_normal((experts, cols)).astype(np.float32)
     dx, dy = cuda.upload(x), cuda.alloc_device(experts * rows * 4)
     K.q4g64_gemv_batch(dptr, 0, dx, cols, dy, rows, cols, group, experts)
-    q = np.stack([nib & 15, nib >> 4], -1).reshape(experts, rows, gpr, group).astype(np.float64) - 8
-    W = (q * s.astype(np.float64)[..., None]).reshape(experts, rows, cols)
+    W = np.stack([O.q4_dequantize(b, rows, cols, group) for b in blobs]).astype(np.float64)
     got = cuda.download(dy, (experts, rows), np.float32)
     for e in range(experts):
         want = W[e] @ x[e].astype(np.float64)
