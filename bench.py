@@ -71,7 +71,7 @@ def measured_traffic(kernel: str, batch: int):
             f = r["fetch_kib"] * r["fetch_factor"] + r["write_kib"] * r["write_factor"]
             return int(round(f * 1024)), r
     return None, "no counter record for this kernel and batch"
-KERNELS = ("lp_moe_router", "lp_moe_route_fused", "lp_moe_route_fused128", "lp_moe_topk_dispatch", "lp_moe_topk", "lp_moe_dispatch", "lp_moe_disp_count",
+KERNELS = ("lp_moe_router", "lp_moe_route_fused", "lp_moe_route_fused128", "lp_moe_topk_dispatch", "lp_moe_topk", "lp_moe_dispatch", "lp_moe_disp_one", "lp_moe_disp_count",
            "lp_moe_disp_scan", "lp_moe_disp_scatter", "lp_moe_ximage", *GATEUP_KERNELS, *DOWN_KERNELS,
            "lp_moe_combine")
 
@@ -230,7 +230,7 @@ def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int) -> dict:
 
 
 PREFILL_T = 2048
-DISPATCH_KERNELS = ("lp_moe_topk", "lp_moe_disp_count", "lp_moe_disp_scan", "lp_moe_disp_scatter")
+DISPATCH_KERNELS = ("lp_moe_topk", "lp_moe_disp_one", "lp_moe_disp_count", "lp_moe_disp_scan", "lp_moe_disp_scatter")
 PREFILL_KERNELS = ("lp_moe_router", "lp_gemm_router", *DISPATCH_KERNELS, "lp_moe_ximage",
                    "lp_gemm_gateup", "lp_gemm_down", "lp_moe_combine")
 MFMA_PEAK_TFLOPS = 2500.0   # MI355X dense fp16 / bf16 MFMA

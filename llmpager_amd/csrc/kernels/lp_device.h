@@ -466,6 +466,25 @@ __device__ __forceinline__ void write_h16_image(const float* row, int cols, uint
     if (threadIdx.x == 0) *exp_out = e;
 }
 
+// The images of token t of a routed batch by one wave: quads of lanes
+// converting sub-groups (digits) or 16-byte words l, l + 64, ... (fp16, after
+// the row's largest magnitude), and W.xexp[t].
+__device__ __forceinline__ void write_ximage(const lpk::RouteArgs& a, int t) {
+    const int H = a.L.hidden, lane = lane_id();
+    const float* row = reinterpret_cast<const float*>(a.x) + (size_t)t * H;
+    if (a.make_xf & lpk::kImgDigits)
+        write_dimage(row, H, reinterpret_cast<uint8_t*>(a.W.xd) + (size_t)t * lpk::dimage_bytes(H), lane, 64);
+    if (a.make_xf & lpk::kImgF16) {
+        const int e = h16_exp(row_absmax_wave(row, H, lane, 64));
+        uint8_t* img = reinterpret_cast<uint8_t*>(a.W.xf) + (size_t)t * lpk::himage_bytes(H);
+        if (a.make_xf & lpk::kImgF16Lo)
+            write_h16_words2(row, H, e, img, img + (size_t)a.T * lpk::himage_bytes(H), lane, 64);
+        else
+            write_h16_words(row, H, e, img, lane, 64);
+        if (lane == 0) reinterpret_cast<int*>(a.W.xexp)[t] = e;
+    }
+}
+
 // Direct-to-LDS copy from inline assembly: lane l's 16 bytes at base + off
 // land at LDS address lds + 16 l (base and lds uniform over the wave: an SGPR
 // pair and M0).  Given the intrinsic instead, the compiler waits for every

@@ -560,12 +560,24 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
 // so every product is exact and the sums are fp32 in the matrix core (the
 // GEMV router's lane order is not kept: its results agree to fp32 rounding).
 // The mid and lo MFMAs run only when some lane's x has such a part (never for
-// bf16-valued activations).  Grid (ceil(T / 16), ceil(E / 32)), 256 threads:
-// the workgroup takes 16 tokens x experts 32 y .. 32 y + 31, wave w the w-th
-// quarter of the hidden dimension (its loads four 32-column steps at a time),
-// and the four partial tiles meet in LDS, summed in wave order.
-extern "C" __global__ void __launch_bounds__(256) lp_gemm_router(const RouteArgs a) {
-    __shared__ f32x4_t part[3][2][64];  // waves 1..3: their two partial C tiles per lane
+// bf16-valued activations).  Grid (ceil(T / 16), ceil(E / 32) and, if the
+// call makes images of x, 16 / kRouterWaves more), kRouterWaves waves: the
+// workgroup takes 16 tokens x experts 32 y .. 32 y + 31, wave w the w-th part
+// of the hidden dimension (its loads four 32-column steps at a time), and the
+// partial tiles meet in LDS, summed in wave order.  The rows of the grid past
+// the experts write the images, a wave per token.  Bound by its waves' chain
+// of loads and, in large batches, by x's split: with four waves and the images
+// in a launch of their own 203 tokens of 2048 took 11.5 + 6.2 us, 2048 tokens
+// 17.4 + 7.3; here 10.3 and 20.7.  Eight steps in flight cost registers the
+// image waves miss (28 us at 2048 tokens).
+extern "C" __global__ void __launch_bounds__(64 * kRouterWaves) lp_gemm_router(const RouteArgs a) {
+    __shared__ f32x4_t part[kRouterWaves - 1][2][64];  // waves 1..: their two partial C tiles per lane
+    const int yi = (int)blockIdx.y - (a.L.experts + 31) / 32;
+    if (yi >= 0) {
+        const int t = (int)blockIdx.x * 16 + yi * kRouterWaves + (int)(threadIdx.x >> 6);
+        if (t < a.T) write_ximage(a, t);
+        return;
+    }
     const int H = a.L.hidden, E = a.L.experts, T = a.T;
     const int lane = lane_id(), wave = threadIdx.x >> 6;
     const int m = lane & 15, kb = lane >> 4;
@@ -608,11 +620,11 @@ extern "C" __global__ void __launch_bounds__(256) lp_gemm_router(const RouteArgs
             c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, wb, c1, 0, 0, 0);
         }
     };
-    // this wave's quarter of the 32-column steps (H is a multiple of 32),
+    // this wave's part of the 32-column steps (H is a multiple of 32),
     // four steps' loads in flight before their MFMAs
     const int ns = H >> 5;
-    const int hend = 32 * ((ns * (wave + 1)) >> 2);
-    int h = 32 * ((ns * wave) >> 2);
+    const int hend = 32 * ((ns * (wave + 1)) / kRouterWaves);
+    int h = 32 * ((ns * wave) / kRouterWaves);
     for (; h + 128 <= hend; h += 128) {
         float4 xa[4], xb[4];
         uint4 wa[4], wb[4];
@@ -636,7 +648,7 @@ extern "C" __global__ void __launch_bounds__(256) lp_gemm_router(const RouteArgs
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
+    for (int w = 0; w < kRouterWaves - 1; ++w) {
         c0 += part[w][0][lane];
         c1 += part[w][1][lane];
     }

@@ -297,26 +297,11 @@ __device__ __forceinline__ void router_rows(const RouteArgs& a) {
 
 extern "C" __global__ void __launch_bounds__(256) lp_moe_router(const RouteArgs a) { router_rows(a); }
 
-// Images of x alone (callers that route from their own logits, and the
-// large-batch router): one wave per token, quads of lanes converting
-// sub-groups (digits) or 16-byte words l, l + 64, ... (fp16, after the row's
-// largest magnitude), and W.xexp[t].  Grid (ceil(T / 4)), 256 threads.
+// Images of x alone (callers that route from their own logits): one wave per
+// token.  Grid (ceil(T / 4)), 256 threads.
 extern "C" __global__ void __launch_bounds__(256) lp_moe_ximage(const RouteArgs a) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= a.T) return;
-    const int H = a.L.hidden, lane = lane_id();
-    const float* row = dptr<const float>(a.x) + (size_t)t * H;
-    if (a.make_xf & kImgDigits)
-        write_dimage(row, H, dptr<uint8_t>(a.W.xd) + (size_t)t * dimage_bytes(H), lane, 64);
-    if (a.make_xf & kImgF16) {
-        const int e = h16_exp(row_absmax_wave(row, H, lane, 64));
-        uint8_t* img = dptr<uint8_t>(a.W.xf) + (size_t)t * himage_bytes(H);
-        if (a.make_xf & kImgF16Lo)
-            write_h16_words2(row, H, e, img, img + (size_t)a.T * himage_bytes(H), lane, 64);
-        else
-            write_h16_words(row, H, e, img, lane, 64);
-        if (lane == 0) dptr<int>(a.W.xexp)[t] = e;
-    }
+    if (t < a.T) write_ximage(a, t);
 }
 
 // ---------------------------------------------------------------------------
@@ -948,6 +933,144 @@ extern "C" __global__ void __launch_bounds__(kDispTok) lp_moe_disp_scatter(const
         } else {
             inv[t * k + j] = -1;
         }
+    }
+}
+
+// The same tables in one launch, for batches whose token masks fit LDS (the
+// host's rule: dispatch_one).  One workgroup of 1024 threads.  Bound by its
+// own chain, not by bytes: picks into LDS (one round of loads), masks of 64
+// tokens per expert, one thread per expert over its masks, then one thread per
+// pick (rank = picks of the masks before + set bits below), as many picks in
+// hand as there are threads.  203 tokens, top 8 of 128: 5.8 us for the three
+// launches' 17.3; 2048 tokens 15.0 for 19.1 and two launches' gaps.
+extern "C" __global__ void __launch_bounds__(1024) lp_moe_disp_one(const RouteArgs a) {
+    extern __shared__ __align__(16) uint8_t sm[];
+    const int E = a.L.experts, k = a.L.top_k, T = a.T;
+    const int nm = (T + 63) >> 6, np = T * k;
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    uint64_t* mask = reinterpret_cast<uint64_t*>(sm);                        // [nm][E]
+    int* tokf = reinterpret_cast<int*>(mask + (size_t)nm * E);               // [E][kEntryToks]
+    int* gsl = tokf + (size_t)E * kEntryToks;                                // [E]
+    int* sh = gsl + E;                                                       // [3][16]
+    uint16_t* off = reinterpret_cast<uint16_t*>(sh + 48);                    // [nm][E]: picks of the masks before
+    int16_t* pick = reinterpret_cast<int16_t*>(off + (((size_t)nm * E + 1) & ~(size_t)1));  // [T][k], -1: none
+    // the picks and the slot table in one round of loads, the clears behind them
+    const int* ids = dptr<const int>(a.W.ids);
+    const int slot = tid < E ? dptr<const int>(a.L.slot_table)[tid] : -1;
+    for (int i0 = 0; i0 < np; i0 += 8 * 1024) {
+        int v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int i = i0 + tid + 1024 * q;
+            v[q] = i < np ? ids[i] : -1;
+        }
+        if (i0 == 0) {
+            for (int i = tid; i < nm * E; i += 1024) mask[i] = 0ull;
+            for (int i = tid; i < E * kEntryToks; i += 1024) tokf[i] = -1;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int i = i0 + tid + 1024 * q;
+            if (i < np) pick[i] = (int16_t)v[q];
+        }
+    }
+    __syncthreads();
+    // pick i is token i / k's: a thread's picks lie 1024 apart
+    const int dt = 1024 / k, dr = 1024 - dt * k;
+    const int ft = tid / k, fr = tid - ft * k;
+    for (int i = tid, t = ft, r = fr; i < np; i += 1024) {
+        const int e = pick[i];
+        if (e >= 0) atomicOr(reinterpret_cast<uint32_t*>(&mask[(size_t)(t >> 6) * E + e]) + ((t >> 5) & 1), 1u << (t & 31));
+        t += dt;
+        r += dr;
+        if (r >= k) {
+            r -= k;
+            ++t;
+        }
+    }
+    __syncthreads();
+    int tot = 0;
+    if (tid < E) {
+#pragma unroll 4
+        for (int m = 0; m < nm; ++m) {
+            off[(size_t)m * E + tid] = (uint16_t)tot;
+            tot += __popcll(mask[(size_t)m * E + tid]);
+        }
+    }
+    const int blocks = a.tile_tokens > 0 ? (tot + a.tile_tokens - 1) / a.tile_tokens : 0;
+    const int xg = wave_incl_scan(tot), xu = wave_incl_scan(tot > 0 ? 1 : 0), xt = wave_incl_scan(blocks);
+    if (lane == 63) {
+        sh[wave] = xg;
+        sh[16 + wave] = xu;
+        sh[32 + wave] = xt;
+    }
+    __syncthreads();
+    int g0 = xg - tot, u = xu - (tot > 0 ? 1 : 0), b0 = xt - blocks, total = 0, nu = 0, ntiles = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const int sg = sh[w], su = sh[16 + w], st = sh[32 + w];
+        g0 += w < wave ? sg : 0;
+        u += w < wave ? su : 0;
+        b0 += w < wave ? st : 0;
+        total += sg;
+        nu += su;
+        ntiles += st;
+    }
+    if (tid < E) gsl[tid] = g0;
+    __syncthreads();
+    int* perm = dptr<int>(a.W.perm);
+    int* inv = dptr<int>(a.W.inv);
+    for (int i = tid, t = ft, r = fr; i < np; i += 1024) {
+        const int e = pick[i];
+        int pos = -1;
+        if (e >= 0) {
+            const uint64_t below = (1ull << (t & 63)) - 1ull;
+            const int rank = off[(size_t)(t >> 6) * E + e] + __popcll(mask[(size_t)(t >> 6) * E + e] & below);
+            pos = gsl[e] + rank;
+            perm[pos] = i;
+            if (rank < kEntryToks) tokf[e * kEntryToks + rank] = t;
+        }
+        inv[i] = pos;
+        t += dt;
+        r += dr;
+        if (r >= k) {
+            r -= k;
+            ++t;
+        }
+    }
+    if (tid < E) {
+        dptr<int>(a.W.gs)[tid] = g0;
+        if (tot > 0) dptr<int>(a.W.uniq)[u] = tid;
+        int* tiles = dptr<int>(a.tiles);
+        for (int b = 0; b < blocks; ++b)
+            if (b0 + b < a.max_tiles) tiles[b0 + b] = (u << 16) | b;
+    }
+    if (tid == 0) {
+        dptr<int>(a.W.gs)[E] = total;
+        dptr<int>(a.W.meta)[0] = nu;
+        dptr<int>(a.W.meta)[1] = 0;
+        if (a.tile_tokens > 0) dptr<int>(a.W.meta)[2] = min(ntiles, a.max_tiles);
+    }
+    write_shared_table(a, tid, 1024);
+    __syncthreads();
+    ExpertEntry* et = dptr<ExpertEntry>(a.W.et);
+    const int maxu = min(np, E);
+    ExpertEntry x;
+    if (tid < E && tot > 0) {
+        x.blob = slot >= 0 ? a.L.arena_base + (uint64_t)slot * a.L.slot_span : 0ull;
+        x.p0 = g0;
+        x.ntok = tot;
+#pragma unroll
+        for (int q = 0; q < kEntryToks; ++q) x.tok[q] = tokf[tid * kEntryToks + q];
+        et[u] = x;
+    }
+    if (tid >= nu && tid < maxu) {  // entries past the unique ones are cleared
+        x.blob = 0ull;
+        x.p0 = 0;
+        x.ntok = 0;
+#pragma unroll
+        for (int q = 0; q < kEntryToks; ++q) x.tok[q] = -1;
+        et[tid] = x;
     }
 }
 

@@ -37,6 +37,8 @@ constexpr int kMaxTopK = 16;           // largest top_k the device router accept
 constexpr int kMaxExperts = 1024;      // largest expert count the device router accepts
 constexpr int kTopkFusedMaxT = 8;      // largest T routed by the one-workgroup top-k + dispatch kernel
 constexpr int kTopkDispatchMaxT = 64;  // largest T dispatched by one workgroup (after the top-k kernel)
+constexpr int kDispOneMaxT = 2048;     // largest T whose dispatch one workgroup may do in one launch
+constexpr int kRouterWaves = 8;        // waves of the large-batch router's workgroup (parts of the hidden dimension)
 constexpr int kDispTok = 256;          // tokens per block of the multi-block dispatch
 constexpr int kMaxPairs = 2;           // token pairs the grouped kernels stage at once
 constexpr int kMaxChunk = 16;          // most MFMA steps (4 sub-groups each) one register chunk holds

@@ -69,6 +69,7 @@ enum Fn {
     kResolve,
     kGemmGateup,
     kGemmDown,
+    kDispOne,
     kDispCount,
     kDispScan,
     kDispScatter,
@@ -141,6 +142,7 @@ const FnSpec kSpecs[kNumFns] = {
     {"lp_moe.hsaco", "lp_moe_topk_dispatch"}, {"lp_basic.hsaco", "lp_expf_wave"},
     {"lp_moe.hsaco", "lp_moe_resolve"},
     {"lp_gemm.hsaco", "lp_gemm_gateup"},   {"lp_gemm.hsaco", "lp_gemm_down"},
+    {"lp_moe.hsaco", "lp_moe_disp_one"},
     {"lp_moe.hsaco", "lp_moe_disp_count"}, {"lp_moe.hsaco", "lp_moe_disp_scan"},
     {"lp_moe.hsaco", "lp_moe_disp_scatter"}, {"lp_gemm.hsaco", "lp_gemm_router"},
     {"lp_moe.hsaco", "lp_moe_dispatch"},   {"lp_moe.hsaco", "lp_moe_route_fused"},
@@ -1245,14 +1247,27 @@ static void set_tiles(const lp_moe_layer_desc* d, RouteArgs& ra) {
     ra.max_tiles = ra.tile_tokens ? max_tiles(d, ra.T, ra.tile_tokens) : 0;
 }
 
+// LDS of lp_moe_disp_one (its carving): masks and offsets of every 64 tokens
+// and expert, the first tokens and group start of each expert, the picks.
+static size_t disp_one_lds(const RouteArgs& ra) {
+    const size_t E = (size_t)ra.L.experts, nm = ((size_t)ra.T + 63) / 64;
+    return nm * E * 8 + E * (kEntryToks + 1) * 4 + 48 * 4 + ((nm * E + 1) & ~(size_t)1) * 2 +
+           (size_t)ra.T * ra.L.top_k * 2;
+}
+
 static int route_tail(lp_ctx* c, const RouteArgs& ra, lp_stream s) {
     const int T = ra.T;
     // up to kTopkFusedMaxT tokens: one workgroup does both (one token per
     // wave); more: the top-k spread over workgroups, then one dispatch
-    // workgroup or, past kTopkDispatchMaxT, the three-launch dispatch
+    // workgroup; past kTopkDispatchMaxT one of 1024 threads as long as the
+    // batch's masks fit its LDS, up to the tokens where its single CU loses to
+    // the three-launch dispatch (top 8 of 128, us: 203 tokens 5.8 against
+    // 17.3, 2048 15.0 against 19.1 + gaps, 4096 26.0 against 23.7 + gaps)
     if (T <= kTopkFusedMaxT) return launch(c, kTopkDispatch, dim3(1), dim3(1024), 0, s, ra);
     if (int r = launch(c, kTopk, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ra)) return r;
     if (T <= kTopkDispatchMaxT) return launch(c, kDispatch, dim3(1), dim3(256), 0, s, ra);
+    if (const size_t lds = disp_one_lds(ra); T <= kDispOneMaxT && lds <= c->max_lds)
+        return launch(c, kDispOne, dim3(1), dim3(1024), lds, s, ra);
     const unsigned nb = (unsigned)((T + kDispTok - 1) / kDispTok);
     if (int r = launch(c, kDispCount, dim3(nb), dim3(kDispTok), 0, s, ra)) return r;
     if (int r = launch(c, kDispScan, dim3(1), dim3(1024), 0, s, ra)) return r;
@@ -1281,10 +1296,11 @@ int lp_moe_route(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t x, int T, uint6
     ra.make_xf = image_kinds(d, T);
     set_tiles(d, ra);
     if (T > kTopkDispatchMaxT) {
-        // large batch: the MFMA router, then the images of x on their own
-        dim3 g((unsigned)((T + 15) / 16), (unsigned)((d->experts + 31) / 32));
-        if (int r = launch(c, kGemmRouter, g, dim3(256), 0, s, ra)) return r;
-        if (int r = launch(c, kXImage, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ra)) return r;
+        // large batch: the MFMA router, with workgroups behind its own for the
+        // images of x (a wave per token)
+        dim3 g((unsigned)((T + 15) / 16),
+               (unsigned)((d->experts + 31) / 32 + (ra.make_xf ? (16 + kRouterWaves - 1) / kRouterWaves : 0)));
+        if (int r = launch(c, kGemmRouter, g, dim3(64 * kRouterWaves), 0, s, ra)) return r;
         return route_tail(c, ra, s);
     }
     if (d->hidden * 4 > kRouteXLds) {
