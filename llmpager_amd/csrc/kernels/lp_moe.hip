@@ -937,7 +937,7 @@ extern "C" __global__ void __launch_bounds__(kDispTok) lp_moe_disp_scatter(const
 }
 
 // The same tables in one launch, for batches whose token masks fit LDS (the
-// host's rule: dispatch_one).  One workgroup of 1024 threads.  Bound by its
+// host's rule: disp_one_lds).  One workgroup of 1024 threads.  Bound by its
 // own chain, not by bytes: picks into LDS (one round of loads), masks of 64
 // tokens per expert, one thread per expert over its masks, then one thread per
 // pick (rank = picks of the masks before + set bits below), as many picks in
