@@ -662,8 +662,9 @@ def run_mla(cuda, s, batches, steps: int) -> dict:
         for i in range(n):
             call(i)
         cuda.sync()
-        split_ms, split_n = cuda.profile_read("lp_mla_split")
-        comb_ms, comb_n = cuda.profile_read("lp_mla_combine")
+        # (the _bal forms where a split of the capacity has several chunks)
+        split_ms, split_n = map(sum, zip(*map(cuda.profile_read, ("lp_mla_split", "lp_mla_split_bal"))))
+        comb_ms, comb_n = map(sum, zip(*map(cuda.profile_read, ("lp_mla_combine", "lp_mla_combine_bal"))))
         cuda.profile(False)
         kv_bytes = B * M_CTX * row_bytes
         split_us = split_ms * 1e3 / max(split_n, 1)

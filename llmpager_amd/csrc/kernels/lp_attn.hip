@@ -511,6 +511,15 @@ extern "C" __global__ void __launch_bounds__(256) lp_attn_combine(const AttnArgs
 //           the B operand comes back column-wise through the transposing
 //           LDS read (ds_read_b64_tr_b16: each 16-lane group reads a 4-row x
 //           16-column block, lane i receiving column i's four values).
+// A workgroup's time is its chain of chunks, and at the capacity's split a
+// batch of shorter sequences leaves part of the workgroups without rows and
+// the others with the longest chain: where a split has several chunks
+// the same workgroups are shared out by the lengths (the _bal kernels,
+// mla_share; kernels of their own, as the test costs the others 0.25 us).
+// 16 sequences of 1,024 to 4,096 rows in caches of 4,096: 29.2 us a call by
+// the capacity's split, 26.7 by lengths; all 4,096 long (the split that the
+// capacity gives): 31.8 and 31.2.  The query's loads of the capacity's
+// sequence go out before the lengths arrive (and again if it is another).
 // The cache rows are read once from HBM.  Each split ends with a partial
 // record {max[16], sum[16], acc[16][c_dim]}; lp_mla_combine merges them.
 // ---------------------------------------------------------------------------
@@ -542,11 +551,37 @@ __device__ __forceinline__ f32x4_t mfma_bf16(const uint4& a, const uint4& b, f32
                                                    c, 0, 0, 0);
 }
 
-template <int STEPS>
+// The sharing by lengths, one sequence per lane (batch <= 64): the fewest
+// chunks `per` for which every sequence's splits of `per` chunks (at least
+// one each) fit the launch's batch x splits workgroups; the capacity's split
+// always fits.  Sequence b's splits, and their records, are [incl - splits,
+// incl) of lane b.  False: no shorter chain than the capacity's split.
+struct MlaShare {
+    int per, splits, incl;
+};
+__device__ __forceinline__ bool mla_share(const MlaBatchArgs& a, int len, MlaShare& o) {
+    const int cap = a.span / kMlaRows, n = a.batch * a.splits;
+    const int chunks = lane_id() < a.batch ? max(1, (min(len, a.max_seq) + kMlaRows - 1) / kMlaRows) : 0;
+    const int total = __builtin_amdgcn_readlane(wave_incl_scan(chunks), 63);
+    for (int per = (total + n - 1) / n; per < cap; ++per) {
+        const int s = (chunks + per - 1) / per, incl = wave_incl_scan(s);
+        if (__builtin_amdgcn_readlane(incl, 63) <= n) {
+            o = {per, s, incl};
+            return true;
+        }
+    }
+    return false;
+}
+
+__device__ __forceinline__ int mla_len(const MlaBatchArgs& a) {
+    return lane_id() < a.batch ? gptr<int>(a.seq_lens)[lane_id()] : 0;
+}
+
+template <int STEPS, bool BAL>
 __device__ __forceinline__ void mla_split_body(const MlaBatchArgs& a) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int QK = 32 * STEPS;
-    const int b = blockIdx.y, sp = blockIdx.x;
+    int b = blockIdx.y, sp = blockIdx.x, span = a.span, rec = b * a.splits + sp;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const int n = lane & 15, kb = lane >> 4;
     const int H = a.heads, CD = a.c_dim;
@@ -559,9 +594,43 @@ __device__ __forceinline__ void mla_split_body(const MlaBatchArgs& a) {
     float* sl = reinterpret_cast<float*>(ct + kMlaRows * rsb);  // [16][64]
     // a length past the cache is cut to the cache (rows beyond max_seq
     // belong to the next sequence, or to no allocation at all)
-    const int seq = min(dptr<const int>(a.seq_lens)[b], a.max_seq);
-    const int p0 = sp * a.span;
-    const int p1 = min(seq, p0 + a.span);
+    int seq;
+    if constexpr (BAL)
+        seq = mla_len(a);
+    else
+        seq = dptr<const int>(a.seq_lens)[b];
+    // the query's loads behind the lengths', before any of them is waited for
+    constexpr int kUnits = (STEPS * 64 + 255) / 256;  // query pieces per thread
+    float4 v4[kUnits][2];
+    auto load_q = [&](int bq) {
+        const uint64_t q = a.q + (uint64_t)bq * H * QK * 4;
+#pragma unroll
+        for (int r = 0; r < kUnits; ++r) {
+            const int u = tid + 256 * r, j = u >> 6, l = u & 63, m = l & 15, k8 = l >> 4;
+            v4[r][0] = v4[r][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (u < STEPS * 64 && m < H) {
+                const LP_GLOBAL float4* src = gptr<float4>(q + ((uint64_t)m * QK + 32 * j + 8 * k8) * 4);
+                v4[r][0] = src[0];
+                v4[r][1] = src[1];
+            }
+        }
+    };
+    load_q(b);
+    if constexpr (BAL) {
+        MlaShare sh;
+        if (mla_share(a, seq, sh)) {
+            const int w = rec, b0 = b;
+            b = __popcll(__ballot(sh.incl <= w));  // 64 past the last split
+            if (b >= a.batch) return;              // the whole workgroup
+            sp = w - (__builtin_amdgcn_readlane(sh.incl, b) - __builtin_amdgcn_readlane(sh.splits, b));
+            span = sh.per * kMlaRows;
+            if (b != b0) load_q(b);
+        }
+        seq = __builtin_amdgcn_readlane(seq, b);
+    }
+    seq = min(seq, a.max_seq);
+    const int p0 = sp * span;
+    const int p1 = min(seq, p0 + span);
     const int nchunks = p1 > p0 ? (p1 - p0 + kMlaRows - 1) / kMlaRows : 0;
     // the query's hi / lo images in A order: step j, lane (m, kb) holds
     // q[m][32 j + 8 kb .. + 7]; heads past H are zero
@@ -666,38 +735,23 @@ __device__ __forceinline__ void mla_split_body(const MlaBatchArgs& a) {
         }
         __syncthreads();  // the chunk's LDS is free for the next one
     };
-    // the query's loads first, then the first chunk's rows: the loads retire
-    // in order, so the query images are made while the rows are in flight
+    // the first chunk's rows behind the query's loads: they retire in order, so
+    // the query images are made while the rows are in flight
     uint4 B0[STEPS];
-    {
-        constexpr int kUnits = (STEPS * 64 + 255) / 256;  // query pieces per thread
-        const uint64_t q = a.q + (uint64_t)b * H * QK * 4;
-        float4 v4[kUnits][2];
+    if (nchunks > 0) load_chunk(B0, 0);
 #pragma unroll
-        for (int r = 0; r < kUnits; ++r) {
-            const int u = tid + 256 * r, j = u >> 6, l = u & 63, m = l & 15, k8 = l >> 4;
-            v4[r][0] = v4[r][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (u < STEPS * 64 && m < H) {
-                const LP_GLOBAL float4* src = gptr<float4>(q + ((uint64_t)m * QK + 32 * j + 8 * k8) * 4);
-                v4[r][0] = src[0];
-                v4[r][1] = src[1];
-            }
-        }
-        if (nchunks > 0) load_chunk(B0, 0);
-#pragma unroll
-        for (int r = 0; r < kUnits; ++r) {
-            const int u = tid + 256 * r;
-            if (u < STEPS * 64) {
-                const float v[8] = {v4[r][0].x, v4[r][0].y, v4[r][0].z, v4[r][0].w,
-                                    v4[r][1].x, v4[r][1].y, v4[r][1].z, v4[r][1].w};
-                split8(v, qhi[u], qlo[u]);
-            }
+    for (int r = 0; r < kUnits; ++r) {
+        const int u = tid + 256 * r;
+        if (u < STEPS * 64) {
+            const float v[8] = {v4[r][0].x, v4[r][0].y, v4[r][0].z, v4[r][0].w,
+                                v4[r][1].x, v4[r][1].y, v4[r][1].z, v4[r][1].w};
+            split8(v, qhi[u], qlo[u]);
         }
     }
     __syncthreads();  // the query images
     for (int c = 0; c < nchunks; ++c) chunk(B0, c);
     // the partial record
-    float* part = dptr<float>(a.part) + ((size_t)b * a.splits + sp) * mla_part_floats(CD);
+    float* part = dptr<float>(a.part) + (size_t)rec * mla_part_floats(CD);
     if (wave == 0 && lane < 16) {
         part[lane] = m_run;
         part[16 + lane] = l_run;
@@ -712,46 +766,64 @@ __device__ __forceinline__ void mla_split_body(const MlaBatchArgs& a) {
     }
 }
 
-}  // namespace
-
-extern "C" __global__ void __launch_bounds__(256) lp_mla_split(const MlaBatchArgs a) {
+template <bool BAL>
+__device__ __forceinline__ void mla_split(const MlaBatchArgs& a) {
     switch (a.qk_dim >> 5) {
-        case 3: mla_split_body<3>(a); break;
-        case 4: mla_split_body<4>(a); break;
-        case 6: mla_split_body<6>(a); break;
-        case 8: mla_split_body<8>(a); break;
-        case 12: mla_split_body<12>(a); break;
-        case 16: mla_split_body<16>(a); break;
-        case 18: mla_split_body<18>(a); break;
-        case 20: mla_split_body<20>(a); break;
+        case 3: mla_split_body<3, BAL>(a); break;
+        case 4: mla_split_body<4, BAL>(a); break;
+        case 6: mla_split_body<6, BAL>(a); break;
+        case 8: mla_split_body<8, BAL>(a); break;
+        case 12: mla_split_body<12, BAL>(a); break;
+        case 16: mla_split_body<16, BAL>(a); break;
+        case 18: mla_split_body<18, BAL>(a); break;
+        case 20: mla_split_body<20, BAL>(a); break;
         default: break;  // the host admits only these widths
     }
 }
+
+}  // namespace
+
+extern "C" __global__ void __launch_bounds__(256) lp_mla_split(const MlaBatchArgs a) { mla_split<false>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_mla_split_bal(const MlaBatchArgs a) { mla_split<true>(a); }
 
 // ctx[b][h][d] from the splits' records.  Grid (heads, batch, c_dim / 64),
 // 256 threads: the weights e^(m_s - M) / sum_s e^(m_s - M) l_s go to LDS once
 // per workgroup, then thread (column d, group g) sums the splits s = g, g + 4,
 // ... of its column (four loads in flight per step) and the four groups'
 // sums meet in LDS.
-extern "C" __global__ void __launch_bounds__(256) lp_mla_combine(const MlaBatchArgs a) {
+namespace {
+
+template <bool BAL>
+__device__ __forceinline__ void mla_combine(const MlaBatchArgs& a) {
     __shared__ float wsh[kMlaMaxSplits];
     __shared__ float red[4];
     __shared__ float part_sum[4][64];
     const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     const int CD = a.c_dim, PF = mla_part_floats(CD);
     const float* base = dptr<const float>(a.part) + (size_t)b * a.splits * PF;
-    const float ms = tid < a.splits ? base[(size_t)tid * PF + h] : -INFINITY;
-    const float ls = tid < a.splits ? base[(size_t)tid * PF + 16 + h] : 0.0f;
+    int splits = a.splits;
+    int len = 0;
+    if constexpr (BAL) len = mla_len(a);
+    auto max_of = [&] { return tid < splits ? base[(size_t)tid * PF + h] : -INFINITY; };
+    auto sum_of = [&] { return tid < splits ? base[(size_t)tid * PF + 16 + h] : 0.0f; };
+    float ms = max_of(), ls = sum_of();  // the capacity's split, in flight beside the lengths
+    if constexpr (BAL) {
+        if (MlaShare sh; mla_share(a, len, sh)) {
+            splits = __builtin_amdgcn_readlane(sh.splits, b);
+            base = dptr<const float>(a.part) + (size_t)(__builtin_amdgcn_readlane(sh.incl, b) - splits) * PF;
+            ms = max_of(), ls = sum_of();
+        }
+    }
     const float M = block_max(ms, red);
     const float w = ms == -INFINITY ? 0.0f : expf(ms - M);
     const float den = block_sum(w * ls, red);
-    if (tid < a.splits) wsh[tid] = w / den;
+    if (tid < splits) wsh[tid] = w / den;
     __syncthreads();
     const int d = blockIdx.z * 64 + (tid & 63), g = tid >> 6;
     const float* col = base + 32 + (size_t)h * CD + d;
     float num = 0.0f;
     int s = g;
-    for (; s + 12 < a.splits; s += 16) {
+    for (; s + 12 < splits; s += 16) {
         const float v0 = col[(size_t)s * PF], v1 = col[(size_t)(s + 4) * PF];
         const float v2 = col[(size_t)(s + 8) * PF], v3 = col[(size_t)(s + 12) * PF];
         num = __builtin_fmaf(wsh[s], v0, num);
@@ -759,10 +831,15 @@ extern "C" __global__ void __launch_bounds__(256) lp_mla_combine(const MlaBatchA
         num = __builtin_fmaf(wsh[s + 8], v2, num);
         num = __builtin_fmaf(wsh[s + 12], v3, num);
     }
-    for (; s < a.splits; s += 4) num = __builtin_fmaf(wsh[s], col[(size_t)s * PF], num);
+    for (; s < splits; s += 4) num = __builtin_fmaf(wsh[s], col[(size_t)s * PF], num);
     part_sum[g][tid & 63] = num;
     __syncthreads();
     if (g == 0)
         dptr<float>(a.ctx)[((size_t)b * a.heads + h) * CD + d] =
             (part_sum[0][tid] + part_sum[1][tid]) + (part_sum[2][tid] + part_sum[3][tid]);
 }
+
+}  // namespace
+
+extern "C" __global__ void __launch_bounds__(256) lp_mla_combine(const MlaBatchArgs a) { mla_combine<false>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_mla_combine_bal(const MlaBatchArgs a) { mla_combine<true>(a); }

@@ -101,6 +101,8 @@ enum Fn {
     kAttnCombine,
     kMlaSplit,
     kMlaCombine,
+    kMlaSplitBal,
+    kMlaCombineBal,
     kRmsNormGemv1,
     kRmsNormGemv2,
     kRmsNormGemv4,
@@ -160,6 +162,7 @@ const FnSpec kSpecs[kNumFns] = {
     {"lp_attn.hsaco", "lp_strided_copy"},  {"lp_attn.hsaco", "lp_attn_split_f32"},
     {"lp_attn.hsaco", "lp_attn_split_f16"}, {"lp_attn.hsaco", "lp_attn_combine"},
     {"lp_attn.hsaco", "lp_mla_split"},     {"lp_attn.hsaco", "lp_mla_combine"},
+    {"lp_attn.hsaco", "lp_mla_split_bal"}, {"lp_attn.hsaco", "lp_mla_combine_bal"},
     {"lp_step.hsaco", "lp_rmsnorm_gemv_c1"}, {"lp_step.hsaco", "lp_rmsnorm_gemv_c2"},
     {"lp_step.hsaco", "lp_rmsnorm_gemv_c4"}, {"lp_step.hsaco", "lp_rmsnorm_gemv_c8"},
     {"lp_step.hsaco", "lp_gemv_add_rmsnorm_c1"}, {"lp_step.hsaco", "lp_gemv_add_rmsnorm_c2"},
@@ -847,9 +850,14 @@ int lp_mla_attn_decode_batch(lp_ctx* c, uint64_t q, uint64_t cache, uint64_t cac
     a.scale = scale;
     a.max_seq = max_seq;
     mla_plan(c, batch, max_seq, &a.splits, &a.span);
-    if (int r = launch(c, kMlaSplit, dim3((unsigned)a.splits, (unsigned)batch), dim3(256), lds, s, a)) return r;
-    return launch(c, kMlaCombine, dim3((unsigned)heads, (unsigned)batch, (unsigned)(c_dim / 64)), dim3(256), 0, s,
-                  a);
+    // splits of several chunks: the kernels share the same workgroups (and
+    // records) out by the lengths instead of the capacity, one sequence per
+    // lane; a sequence's records then stay within kMlaMaxSplits, as batch x
+    // splits is below cus + batch and every sequence keeps one
+    const bool bal = a.span > kMlaRows && batch <= 64 && c->cus <= kMlaMaxSplits;
+    if (int r = launch(c, bal ? kMlaSplitBal : kMlaSplit, dim3((unsigned)a.splits, (unsigned)batch), dim3(256), lds, s, a)) return r;
+    return launch(c, bal ? kMlaCombineBal : kMlaCombine, dim3((unsigned)heads, (unsigned)batch, (unsigned)(c_dim / 64)),
+                  dim3(256), 0, s, a);
 }
 
 // ---- the fused decode step (lp_step.hip) ------------------------------------------

@@ -197,6 +197,25 @@ def test_mla_batch_config5(cuda, K, B, qstd):
     _mla_batch(cuda, K, 16, 576, 512, seqs, 4096, 0.0722, qstd, 100 + B)
 
 
+# Workgroups shared out by the sequences' lengths (splits of several chunks):
+# one sequence and the most that fit the lanes (64), one more (the capacity's
+# split), short and full lengths, exactly as many splits as workgroups, an
+# over-long one; wide rows and narrow ones.
+@pytest.mark.parametrize("heads,qk,cd,ms,seqs,device_seqs", [
+    (4, 96, 64, 17000, [200], None),
+    (4, 96, 64, 17000, [16999], None),
+    (4, 96, 64, 6000, [6000, 1, 64], [9000, 1, 64]),
+    (3, 96, 64, 6000, [700, 6000, 129], None),
+    (4, 96, 64, 600, [1 + (37 * i) % 600 for i in range(64)], None),
+    (4, 96, 64, 600, [600] * 63 + [1], None),
+    (4, 96, 64, 600, [1] * 63 + [600], None),
+    (4, 96, 64, 600, [1 + (37 * i) % 600 for i in range(65)], None),
+    (16, 576, 512, 4096, [1024 + (193 * i) % 3072 for i in range(16)], None),
+    (8, 640, 512, 2500, [2500 - 75 * i for i in range(31)], None)])
+def test_mla_batch_shared_by_lengths(cuda, K, heads, qk, cd, ms, seqs, device_seqs):
+    _mla_batch(cuda, K, heads, qk, cd, seqs, ms, 0.0722, 1.0, ms + len(seqs), device_seqs=device_seqs)
+
+
 # The split kernel's edges: query heads per kv head around its blocks of 8
 # (1, 3, 8, 9, 16), row widths that make 16-byte pieces and that do not (f16:
 # 20; f32: 18), wide rows (fewer rows per chunk), lengths around a chunk of 32
