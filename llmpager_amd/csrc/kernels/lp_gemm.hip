@@ -663,6 +663,35 @@ extern "C" __global__ void __launch_bounds__(64 * kRouterWaves) lp_gemm_router(c
     }
 }
 
+// The tile list of a batch of up to 64 tokens, whose dispatch writes none: for
+// each routed expert u < meta[0], ceil(ntok / kGemmBM) token blocks, as
+// (u << 16) | block; meta[2] = their count.  One workgroup.
+extern "C" __global__ void __launch_bounds__(256) lp_gemm_tiles(const GemmArgs a) {
+    __shared__ int sh[4];
+    const int nu = dptr<const int>(a.W.meta)[0];
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    int* tiles = dptr<int>(a.tiles);
+    int base = 0;
+    for (int u0 = 0; u0 < nu; u0 += 256) {
+        const int u = u0 + tid;
+        const int nb = u < nu ? (load_entry(a.W.et, u).ntok + kGemmBM - 1) / kGemmBM : 0;
+        const int x = wave_incl_scan(nb);  // inclusive scan over the workgroup
+        if (lane == 63) sh[wave] = x;
+        __syncthreads();
+        int wb = 0, tot = 0;
+        for (int w = 0; w < 4; ++w) {
+            wb += w < wave ? sh[w] : 0;
+            tot += sh[w];
+        }
+        const int first = base + wb + x - nb;
+        for (int b = 0; b < nb; ++b)
+            if (first + b < a.max_tiles) tiles[first + b] = (u << 16) | b;
+        base += tot;
+        __syncthreads();
+    }
+    if (tid == 0) dptr<int>(a.W.meta)[2] = min(base, a.max_tiles);
+}
+
 extern "C" __global__ void __launch_bounds__(64 * kGemmWaves) lp_gemm_gateup(const GemmArgs a) {
 #define LP_G(rs) gemm_body<0, rs>(a)
     LP_BY_RS(a.L.group, LP_G)

@@ -67,6 +67,7 @@ enum Fn {
     kTopkDispatch,
     kExpfWave,
     kResolve,
+    kGemmTiles,
     kGemmGateup,
     kGemmDown,
     kDispOne,
@@ -143,7 +144,8 @@ const FnSpec kSpecs[kNumFns] = {
     {"lp_moe.hsaco", "lp_moe_combine"},    {"lp_moe.hsaco", "lp_moe_ximage"},
     {"lp_moe.hsaco", "lp_moe_topk_dispatch"}, {"lp_basic.hsaco", "lp_expf_wave"},
     {"lp_moe.hsaco", "lp_moe_resolve"},
-    {"lp_gemm.hsaco", "lp_gemm_gateup"},   {"lp_gemm.hsaco", "lp_gemm_down"},
+    {"lp_gemm.hsaco", "lp_gemm_tiles"},    {"lp_gemm.hsaco", "lp_gemm_gateup"},
+    {"lp_gemm.hsaco", "lp_gemm_down"},
     {"lp_moe.hsaco", "lp_moe_disp_one"},
     {"lp_moe.hsaco", "lp_moe_disp_count"}, {"lp_moe.hsaco", "lp_moe_disp_scan"},
     {"lp_moe.hsaco", "lp_moe_disp_scatter"}, {"lp_gemm.hsaco", "lp_gemm_router"},
@@ -1059,10 +1061,13 @@ static int image_kinds(const lp_moe_layer_desc* d, int T) {
 
 static uint64_t mid_exps_bytes(uint64_t rows, int inter) { return align256(rows * (uint64_t)(inter / 32) * 4); }
 
-// The tile list of a batch above the decode sizes: blocks of this many tokens
-// of each routed expert (0: no list), at most max_tiles of them.
+// The tile list of the kernels that take a batch's experts in blocks: blocks
+// of this many tokens of each routed expert (0: no list), at most max_tiles of
+// them.  The GEMM needs one whatever the batch (few experts reach its average
+// with a handful of tokens): above 64 tokens the dispatch writes it, else
+// lp_gemm_tiles does.
 static int tile_tokens(const lp_moe_layer_desc* d, int T) {
-    return T <= kTopkDispatchMaxT ? 0 : use_gemm(d, T) ? kGemmBM : use_mid(d, T) ? kMidToks : 0;
+    return use_gemm(d, T) ? kGemmBM : use_mid(d, T) ? kMidToks : 0;
 }
 
 static int max_tiles(const lp_moe_layer_desc* d, int T, int tokens) {
@@ -1250,7 +1255,7 @@ static int check_ws(const lp_moe_layer_desc* d, int T, uint64_t ws, uint64_t ws_
 
 // The tile list the dispatch of a batch above 64 tokens writes.
 static void set_tiles(const lp_moe_layer_desc* d, RouteArgs& ra) {
-    ra.tile_tokens = tile_tokens(d, ra.T);
+    ra.tile_tokens = ra.T > kTopkDispatchMaxT ? tile_tokens(d, ra.T) : 0;
     ra.tiles = ra.W.tiles;
     ra.max_tiles = ra.tile_tokens ? max_tiles(d, ra.T, ra.tile_tokens) : 0;
 }
@@ -1630,6 +1635,8 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         gm.T = T;
         gm.tiles = ga.W.tiles;
         gm.max_tiles = max_tiles(d, T, kGemmBM);
+        if (T <= kTopkDispatchMaxT)
+            if (int r = launch(c, kGemmTiles, dim3(1), dim3(256), 0, s, gm)) return r;
         // gate/up writes act as the down GEMM's fp16 images (+ chunk exponents in W.act)
         gm.a_img = ga.W.xf;
         gm.out = ga.W.actimg;

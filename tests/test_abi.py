@@ -152,6 +152,22 @@ def test_ws_layout_alignment_and_size():
         assert (lay.xd - lay.xf > 0) == (T == 2048)
 
 
+def test_ws_layout_has_room_for_every_tile_list():
+    """Batches whose experts average 16 picks go through the prefill GEMM
+    whatever their size (8 experts top 2 at 64 tokens): its tile list, up to
+    pairs / 128 + min(E, pairs) entries, has a part of its own."""
+    for E, k in [(1, 1), (8, 2), (8, 8), (16, 4), (16, 10), (32, 8), (20, 6), (128, 8)]:
+        for T in range(1, 301):
+            pairs = T * k
+            if pairs < 16 * min(E, pairs):
+                continue
+            lay = lp.ws_layout(lp.LayerDesc(hidden=256, inter=128, experts=E, top_k=k, group=32), T)
+            offs = [getattr(lay, f[0]) for f in lp.WsLayout._fields_ if f[0] != "tiles"]
+            assert lay.tiles not in (lay.actimg, lay.xexp), (E, k, T)
+            room = min(o for o in offs if o > lay.tiles) - lay.tiles
+            assert room >= 4 * (pairs // 128 + min(E, pairs)), (E, k, T)
+
+
 def test_workspace_check_rejects_undersized_workspaces():
     """lp_moe_workspace_check, the pre-launch check of every MoE entry point
     that takes a workspace: null, misaligned and short workspaces are refused

@@ -32,7 +32,7 @@ def _layer_vs_oracle(cuda, L: DeviceLayer, T: int, seed: int, logits=None, sampl
         cuda.free_device(p)
     rows = np.arange(T) if sample is None else np.asarray(sample)
     want = O.moe_layer(L.oracle_desc(), L.oracle_blobs(), x[rows], h[rows].copy(),
-                       logits_in=np.ascontiguousarray(got_logits[rows]), threads=8)[0]
+                       logits_in=np.ascontiguousarray(got_logits[rows]), threads=8, shared_blob=L.shared)[0]
     assert status[1] == 0
     err = rel_l2(got[rows] - h[rows], want - h[rows])
     assert err <= 1e-3, err
@@ -52,6 +52,22 @@ def test_gemm_layer_ragged(cuda, H, I, group):
     # 32-row gate/up block, H = 320 a 64-row down block); group 64 scales
     L = DeviceLayer(cuda, H=H, I=I, E=8, k=3, group=group, seed=22, router_std=0.05)
     _layer_vs_oracle(cuda, L, 100, seed=2)
+    L.free()
+
+
+@pytest.mark.parametrize("H,I,E,k,T,shared", [
+    (256, 128, 8, 2, 64, None), (256, 128, 16, 10, 30, None), (256, 160, 8, 8, 16, None), (320, 128, 32, 8, 64, None),
+    (256, 128, 8, 4, 32, None), (256, 128, 8, 4, 63, None), (256, 128, 16, 8, 65, None), (256, 128, 1, 1, 16, None),
+    (256, 128, 8, 2, 64, (192, 32))])
+def test_gemm_layer_few_experts(cuda, H, I, E, k, T, shared):
+    # few experts reach the GEMM's average per expert in batches that the
+    # decode routing dispatches (up to 64 tokens; 65 beside them): routed by
+    # the layer (one launch for logits, top-k and dispatch) and from logits
+    # (up to 8 tokens would be one workgroup; more, top-k then dispatch)
+    L = DeviceLayer(cuda, H=H, I=I, E=E, k=k, group=32, seed=25, router_std=0.05, shared=shared)
+    logits = (np.random.default_rng(T).standard_normal((T, E)) - 0.4 * np.arange(E)).astype(np.float32)
+    for lg in (None, logits):
+        _layer_vs_oracle(cuda, L, T, seed=T, logits=lg)
     L.free()
 
 
