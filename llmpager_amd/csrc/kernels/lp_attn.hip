@@ -5,8 +5,8 @@
 // over the shared latent cache, batched bf16 GEMV, strided copy), behind
 // 1:1 launchers with the reference's argument meaning.  The arithmetic is
 // this build's own: decode attention is split over positions (one workgroup
-// per (head, split), partial records merged by a second kernel), and config
-// 5's batched MLA decode over bf16 latent caches runs on MFMA.
+// per (block of query heads of a kv head, split), partial records merged by a
+// second kernel), and config 5's batched MLA decode over bf16 latent caches runs on MFMA.
 #include "lp_device.h"
 
 using namespace lp;
@@ -235,67 +235,92 @@ extern "C" __global__ void __launch_bounds__(256) lp_strided_copy(const StridedC
 // One token's attention is a chain of memory round trips, not bytes (3 MB at
 // 1,500 positions of 4 kv heads), so a workgroup brings a chunk of rows'
 // keys and values in by one burst of coalesced loads, fp32 in LDS, and all
-// query heads of the kv head use them: each row is read once for the group.
-//   scores   thread (rows t % 32 and t % 32 + 32, head t / 32): fused
-//            multiply-adds over the row, the rows padded by 16 bytes so 16 lanes' 16-byte reads
-//            cover the banks;
+// query heads of the kv head use them: each row is read once for the group,
+// the next chunk's while this one is worked on.
+//   scores   attn_scores: LDS reads bound it, so each piece serves several
+//            products; the rows are padded by 16 bytes;
 //   softmax  online over the chunks, each head's scores in half a wave;
 //   context  thread (4 columns, kAttnHeads / slots heads): rows from LDS,
-//            probabilities broadcast.
+//            probabilities of four rows at a time, broadcast.
 // One split writes out[h] = acc / sum; more write records {max, sum,
-// acc[out_dim]} that lp_attn_combine merges.  (One thread per key row and a
-// workgroup per query head before: 38.4 us at 32 heads on 4 kv heads, 1,502
-// f16 rows of 128; 11.3 now.  The merge 16.1 before, 4.5 now.)
+// acc[out_dim]} that lp_attn_combine merges.  Measured, whole calls (us),
+// with a thread per key row and a workgroup per query head, with one row and
+// head per thread and chunks loaded when they are needed, and as it is:
+// 32 heads on 4 kv heads of 128 f16, 1,500 rows 35.1, 13.0, 12.7 (100 rows 9.8,
+// 11.0, 9.3); MLA, 16 heads of 576 / 512 in a cache of 4,096 (its scratch
+// holds seven records), 700 rows 40.2, 66.9, 38.8 and 1,500 rows 65.4, 108.9,
+// 61.9.
 // ---------------------------------------------------------------------------
 namespace {
 
-// Rows [0, rows) of a cache at element `at` as fp32 in LDS, row stride rs
-// floats, columns past n zero.  A vector piece is 16 bytes; four pieces per
-// thread are loaded before the first is stored.
-template <bool F16>
+// Rows of a cache from element `at` as fp32 in LDS, row stride rs floats,
+// columns past n zero.  A vector piece is 16 bytes; NP pieces per thread are
+// loaded (load) before the first is stored (store).
+template <bool F16, int NP>
 struct AttnStage {
     static constexpr int kPer = F16 ? 8 : 4;
     uint64_t src;  // address of the first row
     float* dst;
     int row_bytes, rs, n, n4, rows, pieces;
+    int per, dr, dm;  // pieces of a row; 256 pieces further: rows, pieces
+    int r0, m0;       // this thread's first piece not yet stored: row, piece
     bool vec;
-    uint4 u[4];
-    __device__ __forceinline__ AttnStage(float* d, int rs_, uint64_t base, size_t at, int row_stride, int rows_, int n_,
-                                         int n4_)
-        : src(base + at * (F16 ? 2 : 4)), dst(d), row_bytes(row_stride * (F16 ? 2 : 4)), rs(rs_), n(n_), n4(n4_),
-          rows(rows_) {
+    u32x4_t u[NP];
+    __device__ __forceinline__ AttnStage(float* d, int rs_, uint64_t base, size_t at, int row_stride, int n_, int n4_)
+        : src(base + at * (F16 ? 2 : 4)), dst(d), row_bytes(row_stride * (F16 ? 2 : 4)), rs(rs_), n(n_), n4(n4_) {
         vec = (n & (kPer - 1)) == 0 && (src & 15) == 0 && (row_bytes & 15) == 0;
-        pieces = vec ? rows * (n / kPer) : 0;
+        per = max(n / kPer, 1);
+        dr = 256 / per, dm = 256 - dr * per;
+    }
+    // the rows to bring in: rows_ of them, `skip` past those before
+    __device__ __forceinline__ void next(int skip, int rows_) {
+        src += (uint64_t)(uint32_t)skip * (uint32_t)row_bytes;
+        rows = rows_;
+        pieces = vec ? rows * per : 0;
+        r0 = (int)threadIdx.x / per, m0 = (int)threadIdx.x - r0 * per;
+    }
+    __device__ __forceinline__ void step(int& r, int& m) const {
+        r += dr, m += dm;
+        if (m >= per) ++r, m -= per;
     }
     __device__ __forceinline__ void load(int i0) {
-        const int per = n / kPer;
+        int r = r0, m = m0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int i = min(i0 + 256 * j + (int)threadIdx.x, pieces - 1), r = i / per;
-            u[j] = *gptr<uint4>(src + (uint64_t)((uint32_t)r * (uint32_t)row_bytes + 16u * (uint32_t)(i - r * per)));
+        for (int j = 0; j < NP; ++j) {
+            if (i0 + 256 * j >= pieces) break;  // uniform
+            u[j] = *gptr<u32x4_t>(src + (uint64_t)((uint32_t)min(r, rows - 1) * (uint32_t)row_bytes + 16u * (uint32_t)m));
+            step(r, m);
         }
     }
     __device__ __forceinline__ void store(int i0) {
-        const int per = n / kPer;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int i = i0 + 256 * j + (int)threadIdx.x, r = i / per;
-            if (i >= pieces) break;
-            float* o = dst + r * rs + (i - r * per) * kPer;
-            if constexpr (F16) {
-                reinterpret_cast<float4*>(o)[0] =
-                    make_float4(half_bits_to_f32(u[j].x), half_bits_to_f32(u[j].x >> 16), half_bits_to_f32(u[j].y),
-                                half_bits_to_f32(u[j].y >> 16));
-                reinterpret_cast<float4*>(o)[1] =
-                    make_float4(half_bits_to_f32(u[j].z), half_bits_to_f32(u[j].z >> 16), half_bits_to_f32(u[j].w),
-                                half_bits_to_f32(u[j].w >> 16));
-            } else {
-                *reinterpret_cast<uint4*>(o) = u[j];
+        for (int j = 0; j < NP; ++j) {
+            if (i0 + 256 * j >= pieces) break;
+            if (r0 < rows) {
+                float* o = dst + r0 * rs + m0 * kPer;
+                if constexpr (F16) {
+                    reinterpret_cast<float4*>(o)[0] =
+                        make_float4(half_bits_to_f32(u[j][0]), half_bits_to_f32(u[j][0] >> 16), half_bits_to_f32(u[j][1]),
+                                    half_bits_to_f32(u[j][1] >> 16));
+                    reinterpret_cast<float4*>(o)[1] =
+                        make_float4(half_bits_to_f32(u[j][2]), half_bits_to_f32(u[j][2] >> 16), half_bits_to_f32(u[j][3]),
+                                    half_bits_to_f32(u[j][3] >> 16));
+                } else {
+                    *reinterpret_cast<u32x4_t*>(o) = u[j];
+                }
             }
+            step(r0, m0);
         }
     }
-    __device__ __forceinline__ void scalar() {  // widths or addresses that do not make 16-byte pieces
-        for (int i = threadIdx.x; i < rows * 4 * n4; i += 256) {
+    // the whole of it from the second round on (the first is in flight)
+    __device__ __forceinline__ void finish() {
+        store(0);
+        for (int i = 256 * NP; i < pieces; i += 256 * NP) {
+            load(i);
+            store(i);
+        }
+        if (vec) return;
+        for (int i = threadIdx.x; i < rows * 4 * n4; i += 256) {  // no 16-byte pieces
             const int r = i / (4 * n4), c = i - r * 4 * n4;
             const uint64_t row = src + (uint64_t)r * (uint32_t)row_bytes;
             float v = 0.0f;
@@ -310,9 +335,52 @@ struct AttnStage {
     }
 };
 
+// A chunk's scores before their scale, pr[head][row] for rows 0 .. 16 R - 1:
+// thread (part tid % 8, head quad, rg = tid / 16) multiplies the row pieces
+// part, part + 8, ... of rows rg + 16 r with its four heads', so that a piece
+// read from LDS serves R or four products (LDS reads bound this pass).
+template <int R>
+__device__ __forceinline__ void attn_scores(const float* qs, const float* kt, int krs, int d4, float* pr) {
+    static_assert(kAttnHeads == 8, "two quads of heads");
+    const int part = threadIdx.x & 7, h4 = ((threadIdx.x >> 3) & 1) * 4, rg = threadIdx.x >> 4;
+    float acc[4][R];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[h][r] = 0.0f;
+    const float4* q4 = reinterpret_cast<const float4*>(qs) + h4 * d4;
+    for (int i = part; i < d4; i += 8) {
+        float4 k[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) k[r] = reinterpret_cast<const float4*>(kt + (rg + 16 * r) * krs)[i];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const float4 y = q4[h * d4 + i];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                acc[h][r] = __builtin_fmaf(y.x, k[r].x, acc[h][r]);
+                acc[h][r] = __builtin_fmaf(y.y, k[r].y, acc[h][r]);
+                acc[h][r] = __builtin_fmaf(y.z, k[r].z, acc[h][r]);
+                acc[h][r] = __builtin_fmaf(y.w, k[r].w, acc[h][r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float v = acc[h][r];  // over the eight lanes: quad permutations, then the halves of eight
+            v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, false));
+            v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, false));
+            v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));
+            if (part == ((h * R + r) & 7)) pr[(h4 + h) * kAttnRows + rg + 16 * r] = v;
+        }
+}
+
 // HPT: query heads per thread in the context pass (1 up to 128 columns, 2 up
-// to 256, 4 up to 512, 8 up to 1024).
-template <bool F16, int HPT>
+// to 256, 4 up to 512, 8 up to 1024).  NK, NV: pieces of keys and values per
+// thread in flight (18: the whole of an MLA chunk, 32 rows of 576 f32).
+template <bool F16, int HPT, int NK, int NV>
 __device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, sp = blockIdx.y;
@@ -322,14 +390,22 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
     const int d4 = (a.dot_dim + 3) >> 2, o4 = (a.out_dim + 3) >> 2;
     const int krs = attn_row_floats(a.dot_dim), vrs = a.shared_kv ? krs : attn_row_floats(a.out_dim);
     float* qs = reinterpret_cast<float*>(lds);  // [kAttnHeads][4 d4]
-    float* pr = qs + kAttnHeads * 4 * d4;       // [kAttnHeads][32]
+    float* pr = qs + kAttnHeads * 4 * d4;       // [kAttnHeads][kAttnRows]
     float* al = pr + kAttnHeads * kAttnRows;    // [kAttnHeads]: the chunk's rescaling
     float* kt = al + kAttnHeads;                // [rows][krs]
     float* vt = a.shared_kv ? kt : kt + a.rows * krs;
-    const float* q = dptr<const float>(a.q) + (size_t)h0 * a.dot_dim;
-    for (int i = tid; i < kAttnHeads * 4 * d4; i += 256) {
-        const int h = i / (4 * d4), d = i - h * 4 * d4;
-        qs[i] = h < nh && d < a.dot_dim ? q[(size_t)h * a.dot_dim + d] : 0.0f;
+    // the block's query heads: rows of dot_dim floats one behind the other
+    const uint64_t q = a.q + (uint64_t)h0 * (uint32_t)a.dot_dim * 4u;
+    const bool qvec = (a.dot_dim & 3) == 0 && (q & 15) == 0;
+    constexpr int NQ = 8;  // up to 8 heads of 1024 columns by 16-byte pieces
+    float4 qv[NQ];
+    if (qvec) {
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+            const int i = tid + 256 * j;
+            qv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (i < nh * d4) qv[j] = gptr<float4>(q)[i];
+        }
     }
     const size_t kv_off = (size_t)kvh * a.kv_stride;
     const int p0 = sp * a.span, p1 = min(a.seq_len, p0 + a.span);
@@ -341,43 +417,45 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
     float4 acc[HPT];
 #pragma unroll
     for (int j = 0; j < HPT; ++j) acc[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    // a chunk's loads go out before the previous chunk is worked on
+    const size_t at = kv_off + (size_t)p0 * a.row_stride;
+    AttnStage<F16, NK> K(kt, krs, a.k, at, a.row_stride, a.dot_dim, d4);
+    AttnStage<F16, NV> V(vt, vrs, a.v, at, a.row_stride, a.out_dim, o4);
+    auto issue = [&](int skip, int n) {
+        K.next(skip, n);
+        V.next(skip, a.shared_kv ? 0 : n);
+        K.load(0);
+        V.load(0);
+    };
+    issue(0, min(a.rows, p1 - p0));
+    if (qvec) {
+#pragma unroll
+        for (int j = 0; j < NQ; ++j)
+            if (tid + 256 * j < kAttnHeads * d4) reinterpret_cast<float4*>(qs)[tid + 256 * j] = qv[j];
+    } else {
+        for (int i = tid; i < kAttnHeads * 4 * d4; i += 256) {
+            const int h = i / (4 * d4), d = i - h * 4 * d4;
+            qs[i] = h < nh && d < a.dot_dim ? gptr<float>(q)[h * a.dot_dim + d] : 0.0f;
+        }
+    }
     for (int p = p0; p < p1; p += a.rows) {
         const int n = min(a.rows, p1 - p);
         if (p > p0) __syncthreads();  // the previous chunk's rows are read
-        const size_t at = kv_off + (size_t)p * a.row_stride;
-        AttnStage<F16> K(kt, krs, a.k, at, a.row_stride, n, a.dot_dim, d4);
-        AttnStage<F16> V(vt, vrs, a.v, at, a.row_stride, a.shared_kv ? 0 : n, a.out_dim, o4);
-        for (int i = 0; i < max(K.pieces, V.pieces); i += 1024) {  // keys and values in one burst
-            if (i < K.pieces) K.load(i);
-            if (i < V.pieces) V.load(i);
-            if (i < K.pieces) K.store(i);
-            if (i < V.pieces) V.store(i);
-        }
-        if (!K.vec) K.scalar();
-        if (!V.vec) V.scalar();
+        K.finish();
+        V.finish();
         __syncthreads();
-        // rows pl and pl + 32 together: one read of q for two
-        float s0 = -INFINITY, s1 = -INFINITY;
-        if (pl < n) {
-            const float4* kr0 = reinterpret_cast<const float4*>(kt + pl * krs);
-            const float4* kr1 = reinterpret_cast<const float4*>(kt + min(pl + 32, n - 1) * krs);
-            const float4* qr = reinterpret_cast<const float4*>(qs + hl * 4 * d4);
-            s0 = s1 = 0.0f;
-#pragma unroll 8
-            for (int i = 0; i < d4; ++i) {
-                const float4 x0 = kr0[i], x1 = kr1[i], y = qr[i];
-                s0 = __builtin_fmaf(y.x, x0.x, s0);
-                s1 = __builtin_fmaf(y.x, x1.x, s1);
-                s0 = __builtin_fmaf(y.y, x0.y, s0);
-                s1 = __builtin_fmaf(y.y, x1.y, s1);
-                s0 = __builtin_fmaf(y.z, x0.z, s0);
-                s1 = __builtin_fmaf(y.z, x1.z, s1);
-                s0 = __builtin_fmaf(y.w, x0.w, s0);
-                s1 = __builtin_fmaf(y.w, x1.w, s1);
-            }
-            s0 *= a.scale;
-            s1 = pl + 32 < n ? s1 * a.scale : -INFINITY;
-        }
+        if (p + a.rows < p1) issue(a.rows, min(a.rows, p1 - p - a.rows));
+        // partial dot products: rows rg, rg + 16, ... of the chunk against four
+        // heads, every eighth piece of the row; the eight parts meet in lanes
+        if (n > 32)
+            attn_scores<4>(qs, kt, krs, d4, pr);
+        else if (n > 16)
+            attn_scores<2>(qs, kt, krs, d4, pr);
+        else
+            attn_scores<1>(qs, kt, krs, d4, pr);
+        __syncthreads();
+        float s0 = pl < n ? pr[hl * kAttnRows + pl] * a.scale : -INFINITY;
+        float s1 = pl + 32 < n ? pr[hl * kAttnRows + pl + 32] * a.scale : -INFINITY;
         float mx = fmaxf(s0, s1);
 #pragma unroll
         for (int o = 16; o >= 1; o >>= 1) mx = fmaxf(mx, shfl_xor(mx, o));
@@ -401,18 +479,34 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
                 const float f = al[(hs + j * slots) & (kAttnHeads - 1)];
                 acc[j] = make_float4(acc[j].x * f, acc[j].y * f, acc[j].z * f, acc[j].w * f);
             }
-#pragma unroll 8
-            for (int r = 0; r < n; ++r) {
-                const float4 v = *reinterpret_cast<const float4*>(vt + r * vrs + 4 * c);
+            auto add = [&](float4& o, float w, const float4& v) {
+                o.x = __builtin_fmaf(w, v.x, o.x);
+                o.y = __builtin_fmaf(w, v.y, o.y);
+                o.z = __builtin_fmaf(w, v.z, o.z);
+                o.w = __builtin_fmaf(w, v.w, o.w);
+            };
+            const float* vc = vt + 4 * c;
+            int r = 0;
+#pragma unroll 2
+            for (; r + 4 <= n; r += 4) {
+                float4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const float4*>(vc + (r + i) * vrs);
 #pragma unroll
                 for (int j = 0; j < HPT; ++j) {
-                    const float w = pr[((hs + j * slots) & (kAttnHeads - 1)) * kAttnRows + r];
-                    acc[j].x = __builtin_fmaf(w, v.x, acc[j].x);
-                    acc[j].y = __builtin_fmaf(w, v.y, acc[j].y);
-                    acc[j].z = __builtin_fmaf(w, v.z, acc[j].z);
-                    acc[j].w = __builtin_fmaf(w, v.w, acc[j].w);
+                    const float4 w = *reinterpret_cast<const float4*>(
+                        pr + ((hs + j * slots) & (kAttnHeads - 1)) * kAttnRows + r);
+                    add(acc[j], w.x, v[0]);
+                    add(acc[j], w.y, v[1]);
+                    add(acc[j], w.z, v[2]);
+                    add(acc[j], w.w, v[3]);
                 }
             }
+            for (; r < n; ++r)
+#pragma unroll
+                for (int j = 0; j < HPT; ++j)
+                    add(acc[j], pr[((hs + j * slots) & (kAttnHeads - 1)) * kAttnRows + r],
+                        *reinterpret_cast<const float4*>(vc + r * vrs));
         }
     }
     // each head's max and sum to the threads that hold its columns
@@ -440,21 +534,28 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a) {
 
 template <bool F16>
 __device__ __forceinline__ void attn_split(const AttnArgs& a) {
-    const int o4 = (a.out_dim + 3) >> 2;
-    if (o4 <= 32)
-        attn_split_body<F16, 1>(a);
-    else if (o4 <= 64)
-        attn_split_body<F16, 2>(a);
-    else if (o4 <= 128)
-        attn_split_body<F16, 4>(a);
+    if (a.out_dim <= 128)
+        attn_split_body<F16, 1, 8, 8>(a);
     else
-        attn_split_body<F16, 8>(a);
+        attn_split_body<F16, 2, 8, 8>(a);
+}
+
+template <bool F16>
+__device__ __forceinline__ void attn_split_wide(const AttnArgs& a) {
+    if (a.out_dim <= 512)
+        attn_split_body<F16, 4, 18, 8>(a);
+    else
+        attn_split_body<F16, 8, 8, 8>(a);
 }
 
 }  // namespace
 
+// Up to 256 columns of out, and wider rows (kernels of their own: their
+// registers would halve the narrow ones' occupancy).
 extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f32(const AttnArgs a) { attn_split<false>(a); }
 extern "C" __global__ void __launch_bounds__(256) lp_attn_split_f16(const AttnArgs a) { attn_split<true>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_attn_split_wide_f32(const AttnArgs a) { attn_split_wide<false>(a); }
+extern "C" __global__ void __launch_bounds__(256) lp_attn_split_wide_f16(const AttnArgs a) { attn_split_wide<true>(a); }
 
 // Merge of the split records: out[h][d] = sum_s e^(m_s - M) acc_s[d] /
 // sum_s e^(m_s - M) l_s, M = max_s m_s.  Grid (heads, ceil(out_dim / 64)),

@@ -245,7 +245,7 @@ struct StridedCopyArgs {            // kernels.rs:386-404 (strided_copy_f32)
 // `out_dim` wide.  GQA decode has k != v; MLA reads both from its one cache
 // (shared_kv).  A workgroup takes kAttnHeads query heads of one kv head and
 // walks its span in chunks of `rows` (kAttnRows, fewer where the LDS asks).
-constexpr int kAttnSpanMax = 1024;   // more positions than this per record are refused
+constexpr int kAttnSpanMax = 1024;   // a context of more is refused unless the scratch holds a record per this many
 constexpr int kAttnHeads = 8;
 constexpr int kAttnRows = 64;
 constexpr int kAttnMaxSplits = 256;  // lp_attn_combine: one split per thread

@@ -219,7 +219,7 @@ def test_mla_batch_shared_by_lengths(cuda, K, heads, qk, cd, ms, seqs, device_se
 # The split kernel's edges: query heads per kv head around its blocks of 8
 # (1, 3, 8, 9, 16), row widths that make 16-byte pieces and that do not (f16:
 # 20; f32: 18), wide rows (fewer rows per chunk), lengths around a chunk of 32
-# rows, a scratch that holds one record (one split, many chunks), and a cache
+# or 64 rows, a scratch that holds one record (one split, many chunks), and a cache
 # address off 16 bytes.  Bound: a score's fp32 chain is off by at most
 # hd 2^-24 scale sum|q k| (|q k| <= 2: 2 sqrt(hd) hd 2^-24 = 1.7e-4 at
 # hd 128), which moves each probability by that relative amount; the outputs
@@ -247,7 +247,31 @@ def test_attn_decode_edges(cuda, K, f16, heads, kvh, hd, seq, ms, off):
     _free(cuda, dq, dk, dv, dout, dscr)
 
 
-@pytest.mark.parametrize("heads,qk,cd,seq,ms", [(17, 576, 512, 33, 600), (8, 640, 512, 1100, 1100), (1, 30, 18, 40, 64)])
+# Lengths at the edges of a chunk (64 rows, 32 between 65 and 256), of the score
+# pass's 16 rows and of the context pass's 4, with rows that make 16-byte
+# pieces and that do not, up to and past 256 and 512 columns (kernels and
+# register forms of their own), and a query off 16 bytes.  Same bound.
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("heads,kvh,hd,qoff", [(9, 1, 64, 0), (4, 2, 26, 4), (8, 1, 264, 4), (5, 1, 520, 0)])
+@pytest.mark.parametrize("seq", [1, 3, 16, 17, 33, 63, 64, 65, 67, 97, 255, 256, 257, 261])
+def test_attn_decode_chunks(cuda, K, seq, heads, kvh, hd, qoff, f16):
+    ms = 3000
+    rng = np.random.default_rng(hd + seq)
+    scale = 1.0 / np.sqrt(hd)
+    q = _rnd(rng, heads * hd) * 2
+    k, v = (_rnd(rng, kvh * ms * hd).astype(np.float16 if f16 else np.float32) for _ in range(2))
+    dq, dk, dv = cuda.upload(np.concatenate([np.zeros(qoff // 4, np.float32), q])), cuda.upload(k), cuda.upload(v)
+    dout, dscr = cuda.alloc_device(heads * hd * 4), cuda.alloc_device(heads * ms * 4)
+    K.attn_decode(dq + qoff, dk, dv, dout, dscr, heads, kvh, hd, seq, ms, scale, f16)
+    bits = np.uint16 if f16 else np.float32
+    want = O.attn_decode(q, k.view(bits), v.view(bits), heads, kvh, hd, seq, ms, scale, f16)
+    tol = 2.0 * np.sqrt(hd) * hd * 2.0 ** -24
+    assert worst_rel(cuda.download(dout, (heads * hd,), np.float32), want) <= max(tol, 2e-5)
+    _free(cuda, dq, dk, dv, dout, dscr)
+
+
+@pytest.mark.parametrize("heads,qk,cd,seq,ms", [(17, 576, 512, 33, 600), (8, 640, 512, 1100, 1100), (1, 30, 18, 40, 64),
+                                                     (16, 576, 512, 700, 4096), (9, 576, 512, 257, 600)])
 def test_mla_attn_decode_edges(cuda, K, heads, qk, cd, seq, ms):
     rng = np.random.default_rng(seq)
     scale = 1.0 / np.sqrt(qk)
