@@ -1032,12 +1032,26 @@ int lp_attn_block(lp_ctx* c, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm
 
 // ---- fused MoE layer --------------------------------------------------------------
 
+// Whether a blob's regions (gate, up and down of H x I, one group, from their
+// scales to the end of their nibbles) end below `limit` bytes from its base.
+// The balanced, mid-batch and GEMM kernels address them by 32-bit offsets from
+// the blob; the one-shot kernels by 64-bit addresses, so regions further off
+// (a base address that is not the blob's own, say) go through those.
+static bool regions_below(uint64_t limit, int H, int I, int group, uint64_t gate_off, uint64_t up_off,
+                          uint64_t down_off) {
+    const uint64_t cells = (uint64_t)H * (uint64_t)I, bytes = cells / 2 + cells / (uint64_t)std::max(group, 1) * 2;
+    const uint64_t last = std::max({gate_off, up_off, down_off});
+    return last < limit && bytes < limit - last;
+}
+constexpr uint64_t kNear = 1ull << 31;
+
 // Prefill: the grouped GEMM takes over from the decode kernels once routed
 // experts average kGemmMinPairsPerExpert (token, pick) pairs.
 static bool use_gemm(const lp_moe_layer_desc* d, int T) {
     const long pairs = (long)T * d->top_k;
     return pairs >= (long)kGemmMinPairsPerExpert * std::min<long>(d->experts, pairs) &&
-           act_chunks(d->inter) <= kGemmMaxChunks;
+           act_chunks(d->inter) <= kGemmMaxChunks &&
+           regions_below(1ull << 32, d->hidden, d->inter, d->group, d->gate_off, d->up_off, d->down_off);
 }
 
 // Batches between decode and prefill: the routed experts of more than 64
@@ -1055,11 +1069,15 @@ static bool use_mid(const lp_moe_layer_desc* d, int T) {
     const bool balanced = frag_ngp(d->hidden) <= 4 * kGateupChunk && frag_ngp(d->inter) <= 4 * 8 &&
                           scales_in_lds(d->group, d->inter) && maxu <= kBalMaxU &&
                           (pairs + (kBalToks - 1) * maxu) / kBalToks <= 256;
-    return T > kTopkDispatchMaxT && !use_gemm(d, T) && d->slot_span < (1ull << 31) &&
+    return T > kTopkDispatchMaxT && !use_gemm(d, T) &&
+           regions_below(kNear, d->hidden, d->inter, d->group, d->gate_off, d->up_off, d->down_off) &&
            (!balanced || pairs >= kMidMinPairsPerExpert * maxu);
 }
 
-static bool use_mid_shared(const lp_moe_layer_desc* d, int T) { return T > kTopkDispatchMaxT && d->shared_blob; }
+static bool use_mid_shared(const lp_moe_layer_desc* d, int T) {
+    return T > kTopkDispatchMaxT && d->shared_blob &&
+           regions_below(kNear, d->hidden, d->shared_inter, d->shared_group, d->sh_gate_off, d->sh_up_off, d->sh_down_off);
+}
 
 // The images of x a layer's expert kernels read: fp16 images for the prefill
 // GEMM, hi + lo ones for lp_mid.hip, digit images for the grouped kernels.
@@ -1376,7 +1394,10 @@ static bool gateup_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
     const long R = (ga.L.inter + 7) / 8, Rs = nsh ? (ga.L.shared_inter + 7) / 8 : R;
     const bool units_ok = (long)maxv * R + (long)nsh * Rs <= (long)c->cus * std::min(R, Rs);
     return tile_steps_host(H) <= kGateupChunk && maxu + nsh <= kBalMaxU && maxv <= c->cus && units_ok &&
-           (size_t)bal_lds_bytes(H, nw, kBalWaves) <= c->max_lds && ga.L.slot_span < (1ull << 31) &&
+           (size_t)bal_lds_bytes(H, nw, kBalWaves) <= c->max_lds &&
+           regions_below(kNear, H, ga.L.inter, ga.L.group, ga.L.gate_off, ga.L.up_off, 0) &&
+           (!nsh || regions_below(kNear, H, ga.L.shared_inter, ga.L.shared_group, ga.L.sh_gate_off, ga.L.sh_up_off,
+                                  0)) &&
            (uint64_t)pairs * ga.L.inter * 4 < (1ull << 31) &&
            (uint64_t)ga.T * (nsh ? ga.L.shared_inter : 0) * 4 < (1ull << 31);
 }
@@ -1391,6 +1412,7 @@ static bool down_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
     return pairs >= 32 && tile_steps_host(I) <= 8 && scales_in_lds(ga.L.group, I) && maxu <= kBalMaxU &&
            maxv <= c->cus &&
            (size_t)bal_lds_bytes(I, 8 * kDownBalTiles, kBalWaves) <= c->max_lds &&
+           regions_below(kNear, ga.L.hidden, I, ga.L.group, 0, 0, ga.L.down_off) &&
            (uint64_t)pairs * ga.L.hidden * 4 < (1ull << 31);
 }
 
@@ -1669,8 +1691,9 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
                           (size_t)comb_lds(d->inter, Si, sl) <= c->max_lds;
         // the shared MLP's gate/up rides on the routed balanced launch when
         // the groups agree (sh_gu: it did)
-        const int shm =
-            !wave && d->shared_blob && d->shared_group == d->group && !use_mid_shared(d, T) ? shared_entries(T) : 0;
+        // (up to 64 tokens: that launch counts one token group per entry)
+        const int shm = !wave && d->shared_blob && d->shared_group == d->group && T <= kTopkDispatchMaxT
+                            ? shared_entries(T) : 0;
         if (int r = grouped_ffn(c, ga, maxu, true, s, !comb, shm, &sh_gu, &sh_dn)) return r;
         if (comb) {
             const Fn f = !sl ? kDownCombRs : Si <= 8 ? kDownComb : kDownComb16;

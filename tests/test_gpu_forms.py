@@ -93,3 +93,33 @@ def test_decode_kernel_forms(cuda, H, I, group, T, kernels, extra):
         assert np.array_equal(ids[t, :c], wids[t, :c]), t
         assert np.array_equal(wts[t, :c].view(np.uint32), ww[t, :c].view(np.uint32)), t
     assert rel_l2(got - h, want - h) <= 1e-3
+
+
+# Regions 2 GiB and more from the blob's base address (the base lowered, the
+# offsets raised by as much), in the routed slots, the shared blob or both: one
+# token, decode batches that the balanced kernels would take, batches past
+# 64 tokens and the prefill GEMM's sizes all reach them.
+@pytest.mark.parametrize("T,E,k", [(1, 16, 4), (8, 16, 4), (40, 16, 4), (70, 64, 4), (100, 16, 2), (100, 4, 2)])
+@pytest.mark.parametrize("far", [(1 << 33, 0), (0, (1 << 32) - 4096), (1 << 31, 1 << 40)])
+def test_far_regions(cuda, T, E, k, far):
+    H, I, sI = 2048, 768, 256
+    L = DeviceLayer(cuda, H=H, I=I, E=E, k=k, group=32, seed=T, shared=(sI, 32))
+    d = lp.LayerDesc(**{f: getattr(L.desc, f) for f, _ in lp.LayerDesc._fields_})
+    for base, offs, by in (("arena_base", ("gate_off", "up_off", "down_off"), far[0]),
+                           ("shared_blob", ("sh_gate_off", "sh_up_off", "sh_down_off"), far[1])):
+        setattr(d, base, (getattr(d, base) - by) % (1 << 64))
+        for o in offs:
+            setattr(d, o, getattr(d, o) + by)
+    layer = lp.MoeLayer(cuda, d)
+    x, h = fp32_normal(T * H, T).reshape(T, H), np.zeros((T, H), np.float32)
+    lay = lp.ws_layout(d, T)
+    ws, dx, dh = cuda.alloc_device(lay.total), cuda.upload(x), cuda.upload(h)
+    layer.forward(dx, dh, T, ws)
+    got = cuda.download(dh, (T, H), np.float32)
+    glog = cuda.download(ws + lay.logits, (T, E), np.float32)
+    assert layer.status(ws, T)[1] == 0
+    want = O.moe_layer(L.oracle_desc(), L.oracle_blobs(), x, h, logits_in=glog, threads=8, shared_blob=L.shared)[0]
+    assert rel_l2(got, want) <= 1e-3
+    for p in (ws, dx, dh):
+        cuda.free_device(p)
+    L.free()
