@@ -38,8 +38,10 @@
 // through registers into two LDS slots of 128 columns, in operand order with
 // a pad (no bank conflicts either way).
 //
-// act leaves gate/up as hi + lo images with one exponent per (token,
-// sub-group); down scales each staged piece to its row's largest exponent.
+// act leaves gate/up as hi + lo images (2 I bytes each, no padding: together the
+// bytes of the fp32 row that the other kernels keep) with one 16-bit exponent
+// per (token, sub-group); down scales each staged piece to its row's largest
+// exponent.
 #include "lp_device.h"
 
 using namespace lp;
@@ -179,9 +181,13 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
         const int st = min(st0, nst - 1);
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-            R.v[t][0] = *gptr<uint4>(row[t] + 256u * (uint32_t)st);
-            R.v[t][1] = *gptr<uint4>(row[t] + a.lo_off + 256u * (uint32_t)st);
-            if (MODE == 1) R.e[t] = gptr<int>(a.exps)[(size_t)pos[t] * ng + min(4 * st + (piece >> 2), ng - 1)];
+            // x's images end in zero sub-groups, act's rows in the next row:
+            // pieces past their last sub-group repeat it, times zero
+            const int g = 4 * st + (piece >> 2), gc = MODE == 1 && !SV ? min(g, ng - 1) : g;
+            const uint64_t at = row[t] + 64u * (uint32_t)gc;
+            R.v[t][0] = *gptr<uint4>(at);
+            R.v[t][1] = *gptr<uint4>(at + a.lo_off);
+            if (MODE == 1) R.e[t] = gc == g ? gptr<int16_t>(a.exps)[(size_t)pos[t] * ng + gc] : 16 * kExpNone;
         }
     };
     // into the slot (down: times 2^(sub-group exponent - row exponent))
@@ -205,13 +211,13 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
     load_scales(0);
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-        row[t] = a.img + (uint64_t)(uint32_t)pos[t] * a.img_stride + 16u * (uint32_t)piece;
+        row[t] = a.img + (uint64_t)(uint32_t)pos[t] * a.img_stride + 16u * (uint32_t)(piece & 3);
         if (MODE == 0) {
             ex[t] = gptr<int>(a.W.xexp)[pos[t]];
         } else {
             // the row's largest exponent over its 16 lanes
             int m = kExpNone;
-            for (int c = piece; c < ng; c += 16) m = max(m, gptr<int>(a.exps)[(size_t)pos[t] * ng + c]);
+            for (int c = piece; c < ng; c += 16) m = max(m, (int)gptr<int16_t>(a.exps)[(size_t)pos[t] * ng + c]);
 #pragma unroll
             for (int o = 8; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
             ex[t] = m;
@@ -305,7 +311,6 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
         __syncthreads();
         float* ep = reinterpret_cast<float*>(slots) + wave * 64 * kMidEpRow;  // [64 rows][16 tokens]
         const bool live = n0 < NR;
-        const int hb = himage_bytes(NR);
 #pragma unroll
         for (int u = 0; u < TT; ++u) {
 #pragma unroll
@@ -323,7 +328,7 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
             m = fmaxf(m, shfl_xor(m, 16));
             m = fmaxf(m, shfl_xor(m, 32));
             const int ae = m > 0.0f ? h16_exp(m) : 0;
-            if (tt < nt && n0 < 32 * frag_ngp(NR)) {  // padding sub-groups get zeros
+            if (tt < nt && live) {
                 float r[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
@@ -331,10 +336,11 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
                     r[i] = w - (float)(_Float16)w;
                 }
                 const size_t p = (size_t)(x.p0 + tb + tt);
-                LP_GLOBAL uint4* o = gptr_w<uint4>(a.out + p * (2u * (uint32_t)hb) + 2u * (uint32_t)n0);
+                LP_GLOBAL uint4* o = gptr_w<uint4>(a.out + p * (4u * (uint32_t)NR) + 2u * (uint32_t)n0);
                 o[kb] = h16_word(v, ae);
-                o[(hb >> 4) + kb] = h16_word(r, 0);
-                if (live && kb == 0) gptr_w<int>(a.exps)[p * (size_t)(NR >> 5) + (n0 >> 5)] = m > 0.0f ? ae : kExpNone;
+                o[(NR >> 3) + kb] = h16_word(r, 0);
+                if (kb == 0)
+                    gptr_w<int16_t>(a.exps)[p * (size_t)(NR >> 5) + (n0 >> 5)] = (int16_t)(m > 0.0f ? ae : kExpNone);
             }
         }
     } else {
@@ -364,13 +370,13 @@ __device__ __forceinline__ void mid_missing(const MidArgs& a, const ExpertEntry&
     for (int t = tb; t < tb + nt; ++t) {
         const size_t p = (size_t)(x.p0 + t);
         if (MODE == 0) {
-            const int hb = himage_bytes(NR), ng = NR >> 5;
+            const int ng = NR >> 5, g = 4 * chunk + (int)(threadIdx.x & 15) / 4;
             // four sub-groups of 64 bytes, hi and lo
-            if (threadIdx.x < 32)
-                gptr_w<uint4>(a.out + p * (2u * (uint32_t)hb) + (threadIdx.x >> 4) * (uint32_t)hb +
+            if (threadIdx.x < 32 && g < ng)
+                gptr_w<uint4>(a.out + p * (4u * (uint32_t)NR) + (threadIdx.x >> 4) * 2u * (uint32_t)NR +
                               256u * (uint32_t)chunk)[threadIdx.x & 15] = make_uint4(0u, 0u, 0u, 0u);
             if (threadIdx.x < 4 && 4 * chunk + (int)threadIdx.x < ng)
-                gptr_w<int>(a.exps)[p * (size_t)ng + 4 * chunk + threadIdx.x] = kExpNone;
+                gptr_w<int16_t>(a.exps)[p * (size_t)ng + 4 * chunk + threadIdx.x] = (int16_t)kExpNone;
         } else {
             const int r = kMidRows * chunk + (int)threadIdx.x;
             if (r < NR) gptr_w<float>(a.out)[p * NR + r] = 0.0f;

@@ -498,7 +498,7 @@ struct MidArgs {
     uint64_t img_stride; // bytes from one row's image to the next
     uint64_t lo_off;     // bytes from a row's hi image to its lo image
     uint64_t out;        // gate/up: act images, hi and lo per dispatch position; down: y f32
-    uint64_t exps;       // act exponents i32 [position][inter / 32]
+    uint64_t exps;       // act exponents i16 [position][inter / 32]
     uint64_t tiles;      // (entry << 16) | block of kMidToks tokens, meta[2] of them; 0: entry 0's blocks
     int32_t chunks;      // workgroups per block (grid = blocks x chunks)
     int32_t pad0;

@@ -1064,7 +1064,7 @@ static bool use_gemm(const lp_moe_layer_desc* d, int T) {
 // 62.9 + 39.2 here; H 4096 / I 1536, 65 tokens: 429.5 + 145.0 one-shot,
 // 193.4 + 102.6 here).  The shared MLP of every batch above the decode sizes
 // (all T tokens in one entry) goes there too.
-static bool use_mid(const lp_moe_layer_desc* d, int T) {
+static bool want_mid(const lp_moe_layer_desc* d, int T) {
     const long pairs = (long)T * d->top_k, maxu = std::min<long>(d->experts, pairs);
     const bool balanced = frag_ngp(d->hidden) <= 4 * kGateupChunk && frag_ngp(d->inter) <= 4 * 8 &&
                           scales_in_lds(d->group, d->inter) && maxu <= kBalMaxU &&
@@ -1074,28 +1074,9 @@ static bool use_mid(const lp_moe_layer_desc* d, int T) {
            (!balanced || pairs >= kMidMinPairsPerExpert * maxu);
 }
 
-static bool use_mid_shared(const lp_moe_layer_desc* d, int T) {
+static bool want_mid_shared(const lp_moe_layer_desc* d, int T) {
     return T > kTopkDispatchMaxT && d->shared_blob &&
            regions_below(kNear, d->hidden, d->shared_inter, d->shared_group, d->sh_gate_off, d->sh_up_off, d->sh_down_off);
-}
-
-// The images of x a layer's expert kernels read: fp16 images for the prefill
-// GEMM, hi + lo ones for lp_mid.hip, digit images for the grouped kernels.
-static int image_kinds(const lp_moe_layer_desc* d, int T) {
-    const bool gemm = use_gemm(d, T), mid = use_mid(d, T), mid_sh = use_mid_shared(d, T);
-    return (gemm || mid || mid_sh ? kImgF16 : 0) | (mid || mid_sh ? kImgF16Lo : 0) |
-           ((!gemm && !mid) || (d->shared_blob && !mid_sh) ? kImgDigits : 0);
-}
-
-static uint64_t mid_exps_bytes(uint64_t rows, int inter) { return align256(rows * (uint64_t)(inter / 32) * 4); }
-
-// The tile list of the kernels that take a batch's experts in blocks: blocks
-// of this many tokens of each routed expert (0: no list), at most max_tiles of
-// them.  The GEMM needs one whatever the batch (few experts reach its average
-// with a handful of tokens): above 64 tokens the dispatch writes it, else
-// lp_gemm_tiles does.
-static int tile_tokens(const lp_moe_layer_desc* d, int T) {
-    return use_gemm(d, T) ? kGemmBM : use_mid(d, T) ? kMidToks : 0;
 }
 
 static int max_tiles(const lp_moe_layer_desc* d, int T, int tokens) {
@@ -1110,48 +1091,106 @@ static unsigned gemm_grid(const GemmArgs& gm) {
     return (unsigned)((items + kXcds - 1) / kXcds * kXcds);
 }
 
-int lp_moe_ws_layout_get(const lp_moe_layer_desc* d, int T, lp_moe_ws_layout* out) {
-    if (!d || !out || T <= 0) return fail(LP_E_INVALID, "ws layout: bad arguments");
+// Which kernels take a batch's experts, and its workspace.  The parts' sizes
+// are those of the GEMM's or the grouped kernels' buffers; lp_mid.hip's fit
+// inside them (it is taken only where they do), so that a batch between
+// decode and prefill asks for no more than the grouped kernels would:
+//   routed     act images (hi + lo, the bytes of the fp32 rows) in act, their
+//              exponents and the tile list in xd, whose digit images have no
+//              reader then, x's images (hi + lo) in y, which the down
+//              projection writes after their last use (what they need past
+//              its end, xd again);
+//   shared     act images in sh_act; it runs before the routed experts, so
+//              its exponents may sit in a part that those write: act beside
+//              the grouped kernels (x's images in y), y beside the GEMM (x's
+//              lo images behind the hi ones in xf, in xd).
+struct MoePlan {
+    bool gemm, mid, mid_sh;
+    uint64_t sh_exps;  // the shared MLP's act exponents (mid_sh)
+    lp_moe_ws_layout lay;
+
+    // Tokens per block of the routed experts' tile list (0: no list).  The
+    // GEMM needs one whatever the batch (few experts reach its average with a
+    // handful of tokens): above 64 tokens the dispatch writes it, else
+    // lp_gemm_tiles does.
+    int tile_tokens() const { return gemm ? kGemmBM : mid ? kMidToks : 0; }
+    // The images of x the expert kernels read: fp16 images for the GEMM, hi +
+    // lo ones for lp_mid.hip, digit images for the grouped kernels.
+    int image_kinds(const lp_moe_layer_desc* d) const {
+        return (gemm || mid || mid_sh ? kImgF16 : 0) | (mid || mid_sh ? kImgF16Lo : 0) |
+               ((!gemm && !mid) || (d->shared_blob && !mid_sh) ? kImgDigits : 0);
+    }
+};
+
+static MoePlan moe_plan(const lp_moe_layer_desc* d, int T) {
+    MoePlan P{};
+    lp_moe_ws_layout& l = P.lay;
     const uint64_t E = (uint64_t)d->experts, k = (uint64_t)d->top_k, H = (uint64_t)d->hidden,
                    I = (uint64_t)d->inter, t = (uint64_t)T;
+    const bool sh = d->shared_blob != 0;
+    const uint64_t Is = sh ? (uint64_t)d->shared_inter : 0;
+    P.gemm = use_gemm(d, T);
     uint64_t o = 0;
     auto take = [&](uint64_t bytes) {
         uint64_t at = o;
         o = align256(o + bytes);
         return at;
     };
-    out->logits = take(t * E * 4);
-    out->ids = take(t * k * 4);
-    out->wts = take(t * k * 4);
-    out->cnt = take(t * 4);
-    out->gs = take((E + 1) * 4);
-    out->perm = take(t * k * 4);
-    out->inv = take(t * k * 4);
-    out->uniq = take(E * 4);
-    out->meta = take(64);
-    out->et = take(E * sizeof(ExpertEntry));
-    // the prefill GEMM and lp_mid.hip write act as fp16 images (actimg), their exponents here
-    const bool mid = use_mid(d, T), mid_sh = use_mid_shared(d, T);
-    const int kinds = image_kinds(d, T);
-    out->act = take(use_gemm(d, T) ? t * k * (uint64_t)act_chunks((int)I) * 4
-                    : mid          ? mid_exps_bytes(t * k, (int)I)
-                                   : t * k * I * 4);
-    out->y = take(t * k * H * 4);
-    out->xf = take(kinds & kImgF16 ? t * (uint64_t)himage_bytes((int)H) * (kinds & kImgF16Lo ? 2 : 1) : 0);
-    out->xd = take(t * (uint64_t)dimage_bytes((int)H));
-    const bool sh = d->shared_blob != 0;
-    const uint64_t Is = sh ? (uint64_t)d->shared_inter : 0;
-    out->sh_et = take(sh ? (uint64_t)shared_entries(T) * sizeof(ExpertEntry) : 0);
-    out->sh_perm = take(sh ? t * 4 : 0);
-    out->sh_act = take(mid_sh ? mid_exps_bytes(t, (int)Is) + t * 2 * (uint64_t)himage_bytes((int)Is) : t * Is * 4);
-    out->sh_y = take(sh ? t * H * 4 : 0);
-    const bool gemm = use_gemm(d, T);
-    const int tt = tile_tokens(d, T);
-    out->tiles = take(tt ? (uint64_t)max_tiles(d, T, tt) * 4 : 0);
-    out->actimg = take(gemm || mid ? t * k * (uint64_t)himage_bytes((int)I) * (mid ? 2 : 1) : 0);
-    out->xexp = take(t * 4);
-    out->disp = take(T > kTopkDispatchMaxT ? (2 * ((t + kDispTok - 1) / kDispTok) + 1) * E * 4 : 0);
-    out->total = o;
+    l.logits = take(t * E * 4);
+    l.ids = take(t * k * 4);
+    l.wts = take(t * k * 4);
+    l.cnt = take(t * 4);
+    l.gs = take((E + 1) * 4);
+    l.perm = take(t * k * 4);
+    l.inv = take(t * k * 4);
+    l.uniq = take(E * 4);
+    l.meta = take(64);
+    l.et = take(E * sizeof(ExpertEntry));
+    // the prefill GEMM writes act as fp16 images (actimg), their exponents here
+    l.act = take(P.gemm ? t * k * (uint64_t)act_chunks((int)I) * 4 : t * k * I * 4);
+    l.y = take(t * k * H * 4);
+    l.xf = take(P.gemm ? t * (uint64_t)himage_bytes((int)H) : 0);
+    l.xd = take(t * (uint64_t)dimage_bytes((int)H));
+    l.sh_et = take(sh ? (uint64_t)shared_entries(T) * sizeof(ExpertEntry) : 0);
+    l.sh_perm = take(sh ? t * 4 : 0);
+    l.sh_act = take(t * Is * 4);
+    l.sh_y = take(sh ? t * H * 4 : 0);
+    l.tiles = take(P.gemm ? (uint64_t)max_tiles(d, T, kGemmBM) * 4 : 0);
+    l.actimg = take(P.gemm ? t * k * (uint64_t)himage_bytes((int)I) : 0);
+    l.xexp = take(t * 4);
+    l.disp = take(T > kTopkDispatchMaxT ? (2 * ((t + kDispTok - 1) / kDispTok) + 1) * E * 4 : 0);
+    l.total = o;
+    // lp_mid.hip's buffers inside those parts
+    const bool want_sh = want_mid_shared(d, T);
+    const uint64_t img2 = 2 * t * (uint64_t)himage_bytes((int)H), ex_sh = t * (Is / 32) * 2;
+    if (want_mid(d, T) && (want_sh || !sh)) {
+        const uint64_t tiles = std::max(l.xd, align256(l.y + img2));
+        const uint64_t exps = tiles + align256((uint64_t)max_tiles(d, T, kMidToks) * 4);
+        const uint64_t sh_exps = exps + align256(t * k * (I / 32) * 2);
+        if (sh_exps + ex_sh <= l.sh_et) {
+            P.mid = true, P.mid_sh = want_sh;
+            P.sh_exps = sh_exps;
+            l.tiles = tiles;
+            l.actimg = l.act;
+            l.act = exps;
+            l.xf = l.y;
+        }
+    }
+    if (want_sh && P.gemm && ex_sh <= l.xf - l.y) {  // y ends where xf begins
+        P.mid_sh = true;
+        P.sh_exps = l.y;
+    }
+    if (want_sh && !P.gemm && !P.mid && l.y + img2 <= l.xd && ex_sh <= l.y - l.act) {
+        P.mid_sh = true;
+        P.sh_exps = l.act;
+        l.xf = l.y;
+    }
+    return P;
+}
+
+int lp_moe_ws_layout_get(const lp_moe_layer_desc* d, int T, lp_moe_ws_layout* out) {
+    if (!d || !out || T <= 0) return fail(LP_E_INVALID, "ws layout: bad arguments");
+    *out = moe_plan(d, T).lay;
     return LP_OK;
 }
 
@@ -1282,8 +1321,8 @@ static int check_ws(const lp_moe_layer_desc* d, int T, uint64_t ws, uint64_t ws_
 }
 
 // The tile list the dispatch of a batch above 64 tokens writes.
-static void set_tiles(const lp_moe_layer_desc* d, RouteArgs& ra) {
-    ra.tile_tokens = ra.T > kTopkDispatchMaxT ? tile_tokens(d, ra.T) : 0;
+static void set_tiles(const lp_moe_layer_desc* d, const MoePlan& P, RouteArgs& ra) {
+    ra.tile_tokens = ra.T > kTopkDispatchMaxT ? P.tile_tokens() : 0;
     ra.tiles = ra.W.tiles;
     ra.max_tiles = ra.tile_tokens ? max_tiles(d, ra.T, ra.tile_tokens) : 0;
 }
@@ -1334,8 +1373,9 @@ int lp_moe_route(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t x, int T, uint6
     fill_views(d, ws, T, &ra.L, &ra.W);
     ra.x = x;
     ra.T = T;
-    ra.make_xf = image_kinds(d, T);
-    set_tiles(d, ra);
+    const MoePlan P = moe_plan(d, T);
+    ra.make_xf = P.image_kinds(d);
+    set_tiles(d, P, ra);
     if (T > kTopkDispatchMaxT) {
         // large batch: the MFMA router, with workgroups behind its own for the
         // images of x (a wave per token)
@@ -1371,7 +1411,7 @@ int lp_moe_route_logits(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t logits, 
     RouteArgs ra{};
     fill_views(d, ws, T, &ra.L, &ra.W);
     ra.T = T;
-    set_tiles(d, ra);
+    set_tiles(d, moe_plan(d, T), ra);
     if (logits != ra.W.logits)
         HIPCHK(hipMemcpyAsync(reinterpret_cast<void*>(ra.W.logits), reinterpret_cast<void*>(logits),
                               (size_t)T * d->experts * 4, hipMemcpyDeviceToDevice, (hipStream_t)s));
@@ -1581,15 +1621,16 @@ static int mid_ffn(lp_ctx* c, const GroupedArgs& ga, int blocks, uint64_t tiles,
                        m))
         return r;
     m.img = actimg;
-    m.img_stride = 2 * (uint64_t)himage_bytes(I);
-    m.lo_off = (uint64_t)himage_bytes(I);
+    m.img_stride = 4 * (uint64_t)I;  // hi, lo, no padding
+    m.lo_off = 2 * (uint64_t)I;
     m.out = ga.W.y;
     m.chunks = (H + kMidRows - 1) / kMidRows;
     return launch(c, vec(I) ? kMidDown : kMidDownRs, dim3((unsigned)(blocks * m.chunks)), dim3(256), kMidLds, s, m);
 }
 
 // The shared MLP of a batch above the decode sizes: one entry of all T tokens.
-static int mid_shared_ffn(lp_ctx* c, const lp_moe_layer_desc* d, const GroupedArgs& ga, int T, lp_stream s) {
+static int mid_shared_ffn(lp_ctx* c, const lp_moe_layer_desc* d, const GroupedArgs& ga, int T, uint64_t exps,
+                          lp_stream s) {
     GroupedArgs gs = ga;
     gs.L.inter = d->shared_inter;
     gs.L.group = d->shared_group;
@@ -1600,7 +1641,7 @@ static int mid_shared_ffn(lp_ctx* c, const lp_moe_layer_desc* d, const GroupedAr
     gs.W.et = ga.W.sh_et;
     gs.W.perm = ga.W.sh_perm;
     gs.W.y = ga.W.sh_y;
-    return mid_ffn(c, gs, (T + kMidToks - 1) / kMidToks, 0, ga.W.sh_act, ga.W.sh_act + mid_exps_bytes((uint64_t)T, d->shared_inter), s);
+    return mid_ffn(c, gs, (T + kMidToks - 1) / kMidToks, 0, exps, ga.W.sh_act, s);
 }
 
 // The grouped expert kernels and the combine; the fragment images of x are
@@ -1618,12 +1659,13 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
     lp_moe_layer_desc dw = *d0;
     if (wave && !wave_shared) dw.shared_blob = 0;
     const lp_moe_layer_desc* d = &dw;
+    const MoePlan P = moe_plan(d, T);
     if (!have_images) {
         RouteArgs ra{};
         fill_views(d, ws, T, &ra.L, &ra.W);
         ra.x = x;
         ra.T = T;
-        ra.make_xf = image_kinds(d, T);
+        ra.make_xf = P.image_kinds(d);
         if (int r = launch(c, kXImage, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, ra)) return r;
     }
     GroupedArgs ga{};
@@ -1654,7 +1696,11 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         return fail(LP_E_UNSUPPORTED, "hidden/inter too large for one LDS fragment pair");
     ga.pairs_cap = cap;
     bool sh_gu = false, sh_dn = false;  // the shared MLP's gate/up, its down done by the routed launches
-    if (!wave && use_gemm(d, T)) {
+    // the shared MLP of a batch above 64 tokens first: its buffers share the
+    // routed experts' parts of the workspace
+    if (P.mid_sh)
+        if (int r = mid_shared_ffn(c, d, ga, T, ws + P.sh_exps, s)) return r;
+    if (!wave && P.gemm) {
         if ((size_t)kGemmLds > c->max_lds) return fail(LP_E_UNSUPPORTED, "GEMM stages exceed the LDS");
         // the GEMM loads address images and weights as 32-bit offsets from a base
         const uint64_t img_span = std::max((uint64_t)T * himage_bytes(d->hidden),
@@ -1680,7 +1726,7 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
         gm.nblocks = (d->hidden + kGemmBN - 1) / kGemmBN;
         if (int r = launch(c, kGemmDown, dim3(gemm_grid(gm)), dim3(kGemmWaves * 64), 0, s, gm))
             return r;
-    } else if (!wave && use_mid(d, T)) {
+    } else if (!wave && P.mid) {
         if (int r = mid_ffn(c, ga, max_tiles(d, T, kMidToks), ga.W.tiles, ga.W.act, ga.W.actimg, s)) return r;
     } else {
         // one token: down and combine in one launch (after the shared MLP,
@@ -1713,11 +1759,8 @@ static int experts_impl(lp_ctx* c, const lp_moe_layer_desc* d0, uint64_t x, uint
                           lds, s, ga);
         }
     }
-    if (use_mid_shared(d, T)) {
-        if (int r = mid_shared_ffn(c, d, ga, T, s)) return r;
-    } else if (d->shared_blob && !sh_dn) {
+    if (d->shared_blob && !P.mid_sh && !sh_dn)
         if (int r = shared_ffn(c, d, ga, T, s, true, !sh_gu)) return r;
-    }
     return launch(c, kCombine, dim3((unsigned)((d->hidden + 1023) / 1024), (unsigned)T), dim3(256), 0,
                   s, ga);
 }

@@ -168,6 +168,57 @@ def test_ws_layout_has_room_for_every_tile_list():
             assert room >= 4 * (pairs // 128 + min(E, pairs)), (E, k, T)
 
 
+def _align256(n):
+    return (n + 255) // 256 * 256
+
+
+def _decode_or_gemm_bytes(H, I, E, k, T, sI):
+    """A workspace's bytes, as the sum of its parts: the routing tables, then
+    the grouped kernels' buffers (act, y, the digit images of x) or the prefill
+    GEMM's, and the shared MLP's."""
+    ngp = lambda n: 4 * ((n // 32 + 3) // 4)
+    pairs, gemm = T * k, T * k >= 16 * min(E, T * k)
+    parts = [T * E * 4, pairs * 4, pairs * 4, T * 4, (E + 1) * 4, pairs * 4, pairs * 4, E * 4, 64, E * 32,
+             pairs * (ngp(I) // 4 if gemm else I) * 4, pairs * H * 4, T * 64 * ngp(H) if gemm else 0, T * 76 * ngp(H),
+             ((T + 3) // 4 if T <= 64 else 1) * 32 if sI else 0, T * 4 if sI else 0, T * sI * 4, T * H * 4 if sI else 0,
+             (pairs // 128 + min(E, pairs) + 1) * 4 if gemm else 0, pairs * 64 * ngp(I) if gemm else 0, T * 4,
+             (2 * ((T + 255) // 256) + 1) * E * 4 if T > 64 else 0]
+    return sum(map(_align256, parts))
+
+
+def test_ws_layout_between_decode_and_prefill_asks_for_no_more():
+    """The kernels of batches above 64 tokens keep their images, exponents and
+    tile list in parts that the decode kernels or the GEMM need anyway: a
+    workspace holds the same bytes whichever of them run (so one made for a
+    chunk of 279 to 304 tokens takes its 255-token tail), and what is in use at
+    the same time does not overlap."""
+    checked = 0
+    for H, I, E, k, sI in [(2048, 768, 128, 8, 0), (4096, 1536, 128, 8, 0), (2048, 1408, 64, 6, 2816), (160, 96, 16, 2, 0),
+                           (128, 128, 12, 1, 0), (64, 64, 300, 4, 64), (288, 544, 24, 3, 96), (256, 128, 64, 2, 352),
+                           (160, 256, 64, 1, 128), (64, 2048, 1024, 16, 0), (256, 256, 64, 2, 352)]:
+        go, uo, do = lp.blob_offsets(H, I, 32)
+        d = lp.LayerDesc(hidden=H, inter=I, experts=E, top_k=k, group=32, gate_off=go, up_off=uo, down_off=do)
+        if sI:
+            d.shared_blob, d.shared_inter, d.shared_group = 1 << 32, sI, 32
+            d.sh_gate_off, d.sh_up_off, d.sh_down_off = lp.blob_offsets(H, sI, 32)
+        for T in list(range(1, 330)) + [511, 1100, 2048]:
+            lay = lp.ws_layout(d, T)
+            assert lay.total == _decode_or_gemm_bytes(H, I, E, k, T, sI), (H, I, E, k, T)
+            pairs, img = T * k, 64 * 4 * ((H // 32 + 3) // 4)
+            if lay.xf != lay.y or lay.act < lay.y:
+                continue
+            checked += 1  # routed experts by blocks of 32 tokens
+            use = {"tiles": (lay.tiles, 4 * (pairs // 32 + min(E, pairs) + 1)), "exponents": (lay.act, pairs * I // 16),
+                   "act": (lay.actimg, pairs * I * 4)}
+            for name, (at, n) in use.items():
+                for other, (at2, n2) in list(use.items()) + [("y", (lay.y, pairs * H * 4)), ("x", (lay.xf, 2 * T * img)),
+                                                             ("shared", (lay.sh_et, lay.total - lay.sh_et))]:
+                    assert name == other or at + n <= at2 or at2 + n2 <= at, (name, other, H, I, E, k, T)
+    chunk = lp.LayerDesc(hidden=2048, inter=768, experts=128, top_k=8, group=32)
+    assert checked > 500
+    assert lp.ws_layout(chunk, 279).total >= lp.ws_layout(chunk, 255).total
+
+
 def test_workspace_check_rejects_undersized_workspaces():
     """lp_moe_workspace_check, the pre-launch check of every MoE entry point
     that takes a workspace: null, misaligned and short workspaces are refused

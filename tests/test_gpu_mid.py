@@ -117,3 +117,20 @@ def test_mid_shared(cuda, T, E, k, Is, sg):
     gemm = T * k >= 16 * E
     assert err == 0 and rel_l2(got, want) <= (1e-3 if gemm else 1e-4)
     L.free()
+
+
+# ... and where x's images and the shared MLP's exponents sit in parts that the
+# routed experts write after it: beside the balanced decode kernels, in a
+# workspace too small for them (rows short of 128 columns, one pick: the shared
+# MLP through the decode kernels too), and with x's images past y's end
+@pytest.mark.parametrize("H,I,T,E,k,Is", [(256, 256, 70, 64, 2, 352), (160, 256, 70, 64, 1, 128), (288, 96, 100, 10, 1, 160),
+                                          (2048, 1408, 130, 64, 6, 2816)])
+def test_mid_shared_workspace(cuda, H, I, T, E, k, Is):
+    L = DeviceLayer(cuda, H=H, I=I, E=E, k=k, group=32, seed=T + H, shared=(Is, 32))
+    rng = np.random.default_rng(T)
+    x, h = rng.standard_normal((T, H)).astype(np.float32), np.zeros((T, H), np.float32)
+    got, glog, err = _run(cuda, L, x, h)
+    want = O.moe_layer(L.oracle_desc(), L.oracle_blobs(), x, h.copy(), logits_in=glog, threads=8,
+                       shared_blob=L.shared)[0]
+    assert err == 0 and rel_l2(got, want) <= 1e-4
+    L.free()
