@@ -478,6 +478,7 @@ struct GemmArgs {
 // kMidRows rows of down per workgroup of four waves.
 constexpr int kMidToks = 32;
 constexpr int kMidMinPairsPerExpert = 6;
+constexpr int kCus = 256;  // MI355X
 constexpr int kMidRows = 256;
 // LDS: the scales of 64 sub-groups of each of the 256 weight rows (8 bytes of
 // pad: 16 rows' 8-byte reads then cover the banks), two slots of the token

@@ -1054,21 +1054,36 @@ static bool use_gemm(const lp_moe_layer_desc* d, int T) {
            regions_below(1ull << 32, d->hidden, d->inter, d->group, d->gate_off, d->up_off, d->down_off);
 }
 
+static int tile_steps_host(int cols) { return ((cols >> 5) + 3) >> 2; }
+
+// Token groups (kBalToks pairs of one expert) that the balanced kernels may
+// meet with `pairs` picks of up to maxu experts.
+static long bal_groups(long pairs, long maxu) { return std::min(pairs, (pairs + (kBalToks - 1) * maxu) / kBalToks); }
+
+// The shapes that the balanced kernels are built for, whatever the batch: one
+// chunk of K, an expert table they can hold; down with scales in LDS windows.
+static bool bal_gateup_shape(int H, int entries) { return tile_steps_host(H) <= kGateupChunk && entries <= kBalMaxU; }
+static bool bal_down_shape(int I, int group, int entries) {
+    return tile_steps_host(I) <= kDownChunk && scales_in_lds(group, I) && entries <= kBalMaxU;
+}
+
 // Batches between decode and prefill: the routed experts of more than 64
 // tokens go through lp_mid.hip unless the balanced decode kernels take both
-// projections (one chunk of K, no more token groups of four than the card's
-// 256 CUs) and the experts average fewer than kMidMinPairsPerExpert pairs:
-// those re-read no weights for so few tokens (H 2048 / I 768 / 128 experts /
-// top 8: 80 tokens 56.6 + 32.0 us balanced, 63.4 + 39.0 here; past the 256
-// groups the alternative is the one-shot kernels, 81 tokens 104.0 + 56.9,
-// 62.9 + 39.2 here; H 4096 / I 1536, 65 tokens: 429.5 + 145.0 one-shot,
-// 193.4 + 102.6 here).  The shared MLP of every batch above the decode sizes
-// (all T tokens in one entry) goes there too.
+// projections (no more token groups than the card's CUs; the layout is asked
+// for without a context, hence kCus) and the experts average fewer than
+// kMidMinPairsPerExpert pairs.  Whole layers, balanced then lp_mid.hip (us; H
+// 2048 / I 768, 64 experts): 59.1 and 74.7 at 2 pairs per expert, 69.2 and 78.7
+// at 4, 79.4 and 79.9 at 6.2, 95.4 and 83.2 at 9.4.  Beside the one-shot
+// kernels (either projection) the line is lower: equal at 2 for H 4096 / I 1536,
+// at 4 for H 2048 / I 1408 (500 and 387, 170 and 125 at 4 and 9.4).  Below it
+// lp_mid.hip stays: up to a fifth slower there (188 and 212 at 1, H 4096 / I
+// 1536), but its images carry x to 22 bits where the digits of the one-shot
+// kernels carry 16 (errors 1.3e-6 and 2.6e-5).  The shared MLP of every batch
+// above the decode sizes (all T tokens in one entry) goes there too.
 static bool want_mid(const lp_moe_layer_desc* d, int T) {
     const long pairs = (long)T * d->top_k, maxu = std::min<long>(d->experts, pairs);
-    const bool balanced = frag_ngp(d->hidden) <= 4 * kGateupChunk && frag_ngp(d->inter) <= 4 * 8 &&
-                          scales_in_lds(d->group, d->inter) && maxu <= kBalMaxU &&
-                          (pairs + (kBalToks - 1) * maxu) / kBalToks <= 256;
+    const bool balanced = bal_gateup_shape(d->hidden, (int)maxu) && bal_down_shape(d->inter, d->group, (int)maxu) &&
+                          bal_groups(pairs, maxu) <= kCus;
     return T > kTopkDispatchMaxT && !use_gemm(d, T) &&
            regions_below(kNear, d->hidden, d->inter, d->group, d->gate_off, d->up_off, d->down_off) &&
            (!balanced || pairs >= kMidMinPairsPerExpert * maxu);
@@ -1101,9 +1116,10 @@ static unsigned gemm_grid(const GemmArgs& gm) {
 //              projection writes after their last use (what they need past
 //              its end, xd again);
 //   shared     act images in sh_act; it runs before the routed experts, so
-//              its exponents may sit in a part that those write: act beside
-//              the grouped kernels (x's images in y), y beside the GEMM (x's
-//              lo images behind the hi ones in xf, in xd).
+//              the rest may sit in parts that those write: beside the grouped
+//              kernels its exponents in act and x's images at the end of act
+//              and y, beside the GEMM its exponents in y (x's lo images
+//              behind the hi ones in xf, in xd).
 struct MoePlan {
     bool gemm, mid, mid_sh;
     uint64_t sh_exps;  // the shared MLP's act exponents (mid_sh)
@@ -1180,10 +1196,10 @@ static MoePlan moe_plan(const lp_moe_layer_desc* d, int T) {
         P.mid_sh = true;
         P.sh_exps = l.y;
     }
-    if (want_sh && !P.gemm && !P.mid && l.y + img2 <= l.xd && ex_sh <= l.y - l.act) {
+    if (want_sh && !P.gemm && !P.mid && align256(l.act + ex_sh) + align256(img2) <= l.xd) {
         P.mid_sh = true;
         P.sh_exps = l.act;
-        l.xf = l.y;
+        l.xf = l.xd - align256(img2);
     }
     return P;
 }
@@ -1418,22 +1434,20 @@ int lp_moe_route_logits(lp_ctx* c, const lp_moe_layer_desc* d, uint64_t logits, 
     return route_tail(c, ra, s);
 }
 
-static int tile_steps_host(int cols) { return ((cols >> 5) + 3) >> 2; }
-
 // Whether lp_moe_gateup_bal takes the gate/up of ga's routed experts: one
 // chunk of K, an expert table it can hold, no more token groups (up to
 // kBalToks = 4 tokens of one expert each) than CUs, and its LDS.
 static bool gateup_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
     const int H = ga.L.hidden, pairs = ga.T * ga.L.top_k;
-    const int maxv = std::min(pairs, (pairs + (kBalToks - 1) * maxu) / kBalToks);
+    const long maxv = bal_groups(pairs, maxu);
     const int nw = tile_steps_host(H) > 8 ? 16 : 8;
     // with the shared MLP's entries (one token group each): at most the
     // grid's worth of units of the shorter width per workgroup, so that a
     // range still touches at most two blocks
     const int nsh = ga.sh_maxu;
     const long R = (ga.L.inter + 7) / 8, Rs = nsh ? (ga.L.shared_inter + 7) / 8 : R;
-    const bool units_ok = (long)maxv * R + (long)nsh * Rs <= (long)c->cus * std::min(R, Rs);
-    return tile_steps_host(H) <= kGateupChunk && maxu + nsh <= kBalMaxU && maxv <= c->cus && units_ok &&
+    const bool units_ok = maxv * R + (long)nsh * Rs <= (long)c->cus * std::min(R, Rs);
+    return bal_gateup_shape(H, maxu + nsh) && maxv <= c->cus && units_ok &&
            (size_t)bal_lds_bytes(H, nw, kBalWaves) <= c->max_lds &&
            regions_below(kNear, H, ga.L.inter, ga.L.group, ga.L.gate_off, ga.L.up_off, 0) &&
            (!nsh || regions_below(kNear, H, ga.L.shared_inter, ga.L.shared_group, ga.L.sh_gate_off, ga.L.sh_up_off,
@@ -1448,9 +1462,7 @@ static bool gateup_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
 // pairs the one-shot kernel is faster: too few units to share.
 static bool down_balanced(const lp_ctx* c, const GroupedArgs& ga, int maxu) {
     const int I = ga.L.inter, pairs = ga.T * ga.L.top_k;
-    const int maxv = std::min(pairs, (pairs + (kBalToks - 1) * maxu) / kBalToks);
-    return pairs >= 32 && tile_steps_host(I) <= 8 && scales_in_lds(ga.L.group, I) && maxu <= kBalMaxU &&
-           maxv <= c->cus &&
+    return pairs >= 32 && bal_down_shape(I, ga.L.group, maxu) && bal_groups(pairs, maxu) <= c->cus &&
            (size_t)bal_lds_bytes(I, 8 * kDownBalTiles, kBalWaves) <= c->max_lds &&
            regions_below(kNear, ga.L.hidden, I, ga.L.group, 0, 0, ga.L.down_off) &&
            (uint64_t)pairs * ga.L.hidden * 4 < (1ull << 31);

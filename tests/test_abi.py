@@ -219,6 +219,18 @@ def test_ws_layout_between_decode_and_prefill_asks_for_no_more():
     assert lp.ws_layout(chunk, 279).total >= lp.ws_layout(chunk, 255).total
 
 
+@pytest.mark.parametrize("H,I,E,k,T,group", [
+    (2048, 768, 64, 4, 96, 32),     # both projections balanced below: 6 pairs per expert
+    (2048, 768, 128, 8, 81, 32),    # more token groups than CUs
+    (2048, 1408, 64, 2, 65, 32),    # down one-shot: decode batches end at 64 tokens
+    (4096, 1536, 64, 8, 65, 32)])
+def test_mid_batches_begin_at(H, I, E, k, T, group):
+    """Which kernels a batch between decode and prefill takes, as its layout
+    shows it (x's images in y, the act exponents behind it)."""
+    d = lp.LayerDesc(hidden=H, inter=I, experts=E, top_k=k, group=group)
+    assert [(lay.xf == lay.y and lay.act > lay.y) for lay in (lp.ws_layout(d, T - 1), lp.ws_layout(d, T))] == [False, True]
+
+
 def test_workspace_check_rejects_undersized_workspaces():
     """lp_moe_workspace_check, the pre-launch check of every MoE entry point
     that takes a workspace: null, misaligned and short workspaces are refused

@@ -120,9 +120,9 @@ def test_mid_shared(cuda, T, E, k, Is, sg):
 
 
 # ... and where x's images and the shared MLP's exponents sit in parts that the
-# routed experts write after it: beside the balanced decode kernels, in a
-# workspace too small for them (rows short of 128 columns, one pick: the shared
-# MLP through the decode kernels too), and with x's images past y's end
+# routed experts write after it: beside the balanced decode kernels (with rows
+# short of 128 columns and one pick, x's images begin in act), and beside
+# routed experts of this path with x's images past y's end
 @pytest.mark.parametrize("H,I,T,E,k,Is", [(256, 256, 70, 64, 2, 352), (160, 256, 70, 64, 1, 128), (288, 96, 100, 10, 1, 160),
                                           (2048, 1408, 130, 64, 6, 2816)])
 def test_mid_shared_workspace(cuda, H, I, T, E, k, Is):
