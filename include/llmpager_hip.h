@@ -158,7 +158,11 @@ int lp_gemv_add_rmsnorm(lp_ctx* ctx, uint64_t w, uint64_t x, int rows, int cols,
  * fp16 caches [kv_heads, max_seq, 128] at pos, and attn_decode over
  * positions 0..pos into out [heads, 128] (decode.rs:283-294).  q, k and v
  * are read only; scratch [heads, max_seq] f32.  heads / kv_heads in
- * {1, 2, 4, 8, 16}, kv_heads <= 16. */
+ * {1, 2, 4, 8, 16}, kv_heads <= 16.  With more than one split of the context
+ * it uses the stream's arrival counters, like lp_gemv_add_rmsnorm; with more
+ * than 32 (contexts past 2,048 positions whose scratch holds the records) each
+ * query head's merge also waits for its splits, a bounded wait: see
+ * lp_step_errors_sync. */
 int lp_attn_fused(lp_ctx* ctx, uint64_t q, uint64_t k, uint64_t v, uint64_t q_norm, uint64_t k_norm, float eps,
                   float rope_base, uint64_t kcache, uint64_t vcache, uint64_t out, uint64_t scratch, int heads,
                   int kv_heads, int head_dim, int pos, int max_seq, float scale, lp_stream s);
@@ -171,11 +175,14 @@ int lp_attn_block(lp_ctx* ctx, uint64_t q, uint64_t k, uint64_t v, uint64_t q_no
                   float rope_base, uint64_t kcache, uint64_t vcache, uint64_t att, uint64_t scratch, int heads,
                   int kv_heads, int head_dim, int pos, int max_seq, float scale, uint64_t wo, uint64_t h,
                   uint64_t post_ln, uint64_t hn, int hidden, lp_stream s);
-/* The o projection's wait in lp_attn_block is bounded (about 30 ms): one
- * that gives up counts itself and lets the launch end with a wrong result
- * instead of hanging.  This waits for the device, returns the count since the
- * last call in *timeouts (0 normally) and clears it, with the fused step's
- * counters of each stream that had one. */
+/* The waits inside a launch (the o projection's in lp_attn_block, the merges'
+ * of more than 32 splits in lp_attn_fused and lp_attn_block) are bounded (about
+ * 30 ms): one that gives up counts itself and lets the launch end with a wrong
+ * result instead of hanging, and may leave that stream's counters wrong for
+ * the launches after it.  This waits for the device, returns the count since
+ * the last call in *timeouts (0 normally) and clears it, with the fused step's
+ * counters of each stream that had one; results since a call that returned 0
+ * are good if it returns 0 again. */
 int lp_step_errors_sync(lp_ctx* ctx, int32_t* timeouts);
 
 /* ---- MLA absorbed decode: kernels::Kernels (kernels.rs; mla.cu) ----------- */

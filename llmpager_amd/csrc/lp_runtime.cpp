@@ -241,7 +241,7 @@ struct lp_ctx {
     hipStream_t cap_stream = nullptr;         // a capture in progress on this stream ...
     int cap_slot = -1;                        // ... routes through this (the graph's) slot
     bool cap_prof = false;                    // lp_graph_capture_begin: the profiling switch to restore
-    int step_spin = kStepSpinMax;             // polls before lp_attn_block's wait gives up
+    int step_spin = kStepSpinMax;             // polls before a wait of lp_attn_block or lp_attn_fused gives up
     // decode gate/up through lp_moe_gateup_bal (LLMPAGER_HIP_GATEUP_BAL=0 at
     // lp_init turns it off, for comparison)
     bool gateup_bal = true;
