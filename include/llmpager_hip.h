@@ -257,7 +257,11 @@ typedef struct lp_moe_layer_desc {
     uint64_t sh_gate_off, sh_up_off, sh_down_off; /* region offsets in that blob */
 } lp_moe_layer_desc;
 
-/* Byte offsets of the workspace parts for T tokens (all 256-byte aligned). */
+/* Byte offsets of the workspace parts for T tokens (all 256-byte aligned).
+ * Between the decode batches (64 tokens) and the prefill GEMM the parts share
+ * memory, each only with what is not in use at the same time: the routing
+ * tables (logits to et, sh_et, sh_perm) always have theirs, y holds the
+ * routed experts' outputs after the call and x's images before. */
 typedef struct lp_moe_ws_layout {
     uint64_t logits;  /* f32 [T, E] router logits */
     uint64_t ids;     /* i32 [T, k] picked expert ids in pick order, -1 past cnt */
@@ -269,20 +273,23 @@ typedef struct lp_moe_ws_layout {
     uint64_t uniq;    /* i32 [E] experts with picks, ascending */
     uint64_t meta;    /* i32 [16]: [0] unique count, [1] error flags */
     uint64_t et;      /* 32-byte expert entries [E] for the grouped kernels */
-    uint64_t act;     /* f32 [T*k, I]; on the prefill GEMM path i32 [T*k][ceil(I/128)], the
-                         exponent of each 128-column chunk of the act images in actimg */
+    uint64_t act;     /* f32 [T*k, I]; where act is kept as fp16 images (actimg), their exponents:
+                         i32 [T*k][ceil(I/128)] one per 128 columns (prefill GEMM), i16
+                         [T*k][I/32] one per 32 (between decode and prefill) */
     uint64_t y;       /* f32 [T*k, H] */
-    uint64_t xf;      /* [T] fp16 images of x for the prefill GEMM, each row scaled by 2^-xexp[t]
-                         (size 0 without it) */
+    uint64_t xf;      /* [T] fp16 images of x, each row scaled by 2^-xexp[t], for the prefill GEMM;
+                         for a batch of more than 64 tokens below it (and the shared MLP
+                         above 64) with the images of their rounding behind them */
     uint64_t xd;      /* [T] digit images of x for the grouped kernels (per 32 columns 16-bit
                          fixed point as two int8 digits, a seed and a scale) */
     uint64_t sh_et;   /* shared MLP: its expert entry (size 0 without one) */
     uint64_t sh_perm; /* shared MLP: i32 [T] identity token list */
-    uint64_t sh_act;  /* shared MLP: f32 [T, shared_inter] */
+    uint64_t sh_act;  /* shared MLP: f32 [T, shared_inter], above 64 tokens as fp16 images */
     uint64_t sh_y;    /* shared MLP: f32 [T, H] */
-    uint64_t tiles;   /* prefill GEMM tile list (size 0 on the decode path) */
-    uint64_t actimg;  /* prefill GEMM: fp16 images of the act rows (size 0 on the decode path) */
-    uint64_t xexp;    /* i32 [T]: prefill GEMM: the power-of-two exponent of each token's image in xf */
+    uint64_t tiles;   /* tile list of the prefill GEMM and of batches below it (size 0 on the decode
+                         path): (entry << 16) | block, their number in meta[2] */
+    uint64_t actimg;  /* their fp16 images of the act rows (size 0 on the decode path) */
+    uint64_t xexp;    /* i32 [T]: the power-of-two exponent of each token's image in xf */
     uint64_t disp;    /* dispatch scratch of batches above 64 tokens */
     uint64_t total;   /* bytes */
 } lp_moe_ws_layout;

@@ -177,7 +177,7 @@ __device__ __forceinline__ LP_GLOBAL T* gptr_w(uint64_t a) {
 //     16 per lane: words w0..w3 = columns 0-7, 8-15, 16-23, 24-31); MFMA h
 //     (0, 1) takes w & 0x0F0F0F0F and (w >> 4) & 0x0F0F0F0F of words 2h and
 //     2h + 1, i.e. byte t of the lane's 16 holds column
-//     16h + 8 (t >> 3) + 2 (t & 3) + ((t >> 2) & 1)  (digit_col).
+//     16h + 8 (t >> 3) + 2 (t & 3) + ((t >> 2) & 1).
 //   A (activations): row m = 4*slot + th, th = 2*token + digit (0 = hi, 1 =
 //     lo).  Element (m, k = 16*kbA + t) is non-zero only when slot == kbA, so
 //     the 16 output rows keep four sub-groups x four (token, digit) apart.
@@ -233,11 +233,6 @@ __device__ __forceinline__ float* sig_ptr(const Frags& F, int p, int g) {
 __device__ __forceinline__ void zero_block(const Frags& F, int tid, int nthreads) {
     for (int i = tid; i < lpk::kZeroBytes / 16; i += nthreads)
         reinterpret_cast<uint4*>(F.lds)[i] = make_uint4(0, 0, 0, 0);
-}
-
-// Column (within a 32-column sub-group) of digit byte t of MFMA h.
-__device__ __forceinline__ constexpr int digit_col(int h, int t) {
-    return 16 * h + 8 * (t >> 3) + 2 * (t & 3) + ((t >> 2) & 1);
 }
 
 // The largest magnitude below which a sub-group's digits are all zero (its
@@ -721,7 +716,7 @@ __device__ __forceinline__ ABase abase(const Frags& F, int p, int c0) {
     return b;
 }
 
-// The two B operands of one 16-byte nibble load: bytes in digit_col order.
+// The two B operands of one 16-byte nibble load, bytes in operand order.
 __device__ __forceinline__ void q4_digits(const uint4& w, i32x4_t& b0, i32x4_t& b1) {
     b0 = i32x4_t{(int)(w.x & 0x0F0F0F0Fu), (int)((w.x >> 4) & 0x0F0F0F0Fu), (int)(w.y & 0x0F0F0F0Fu),
                  (int)((w.y >> 4) & 0x0F0F0F0Fu)};

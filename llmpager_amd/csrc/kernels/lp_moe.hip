@@ -1903,20 +1903,23 @@ __device__ __forceinline__ void down_group(const Frags& F, WRegs<NS, SL> (&D)[TW
 }
 
 // The matrices and tables one workgroup of the one-shot down works on: the
-// routed experts', or (lp_moe_down_wide's workgroups from sh_wg0 on) the
-// shared MLP's.
+// launch's own, or (lp_moe_down_wide's workgroups from sh_wg0 on) the shared
+// MLP's beside them.
 struct DownView {
     uint64_t et, act, y, down_off;
     int inter, group, wg;  // wg: the workgroup's index among its own kind
-    bool routed;
 };
 
-__device__ __forceinline__ DownView down_view(const GroupedArgs& a) {
+__device__ __forceinline__ DownView own_view(const GroupedArgs& a) {
+    return DownView{a.W.et, a.W.act, a.W.y, a.L.down_off, a.L.inter, a.L.group, (int)blockIdx.x};
+}
+
+__device__ __forceinline__ DownView wide_view(const GroupedArgs& a) {
     const int b = (int)blockIdx.x;
     if (a.sh_wg0 > 0 && b >= a.sh_wg0)
         return DownView{a.W.sh_et, a.W.sh_act, a.W.sh_y, a.L.sh_down_off, a.L.shared_inter, a.L.shared_group,
-                        b - a.sh_wg0, false};
-    return DownView{a.W.et, a.W.act, a.W.y, a.L.down_off, a.L.inter, a.L.group, b, true};
+                        b - a.sh_wg0};
+    return own_view(a);
 }
 
 template <int TW, int NS, bool ONE, int RS, bool SL>
@@ -2051,7 +2054,7 @@ lp_moe_down_bal6(const GroupedArgs a) {
 // picks this kernel only for those), loaded in one piece.
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lp_moe_down(const GroupedArgs a) {
-    const DownView V = down_view(a);
+    const DownView V = own_view(a);
     if (scales_in_lds(V.group, V.inter)) {
         // a 6-step tile (inter 768) loads only its own 6 steps
         if (tile_steps(V.inter) == 6)
@@ -2073,7 +2076,7 @@ lp_moe_down(const GroupedArgs a) {
 // idle on their own).
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lp_moe_down_wide(const GroupedArgs a) {
-    const DownView V = down_view(a);
+    const DownView V = wide_view(a);
     const int S = tile_steps(V.inter);
     if (S <= kDownWideChunk) {
         // tiles of 9..12 steps (inter 1152..1536) load 12 steps, not 16

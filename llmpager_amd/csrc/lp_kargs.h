@@ -346,17 +346,20 @@ struct Workspace {
     uint64_t uniq;       // i32 [E] experts with picks, ascending
     uint64_t meta;       // i32 [16]: [0] = unique count, [1] = error flags
     uint64_t et;         // ExpertEntry [E]
-    uint64_t act;        // f32 [T * k, I] expert-major activations; prefill GEMM: i32 [T * k][act_chunks(I)] act image exponents
+    uint64_t act;        // f32 [T * k, I] expert-major activations; the act images' exponents of the prefill GEMM (i32
+                         // [T * k][act_chunks(I)]) and lp_mid.hip (i16 [T * k][I / 32])
     uint64_t y;          // f32 [T * k, H] expert-major expert outputs
-    uint64_t xf;         // [T] fp16 images of the layer input for the prefill GEMM (himage_bytes(H) each)
+    uint64_t xf;         // [T] fp16 images of the layer input (himage_bytes(H) each): the prefill GEMM's or lp_mid.hip's
+                         // hi ones, whose lo images follow them
     uint64_t xd;         // [T] digit images of the layer input for the grouped kernels (dimage_bytes(H) each)
     uint64_t sh_et;      // shared MLP: shared_entries(T) ExpertEntry (consecutive tokens)
     uint64_t sh_perm;    // shared MLP: i32 [T], t
-    uint64_t sh_act;     // shared MLP: f32 [T, shared_inter]
+    uint64_t sh_act;     // shared MLP: f32 [T, shared_inter]; lp_mid.hip: its act images (4 shared_inter bytes each)
     uint64_t sh_y;       // shared MLP: f32 [T, H]
     uint64_t tiles;      // prefill GEMM and lp_mid.hip: i32 tile list
-    uint64_t actimg;     // prefill GEMM: [T*k] fp16 images of act rows (himage_bytes(I) each)
-    uint64_t xexp;       // prefill GEMM: i32 [T], token t's image exponent in xf
+    uint64_t actimg;     // [T*k] fp16 images of act rows: the prefill GEMM's (himage_bytes(I) each), lp_mid.hip's hi and
+                         // lo (4 I bytes together)
+    uint64_t xexp;       // i32 [T], token t's image exponent in xf
     uint64_t disp;       // multi-block dispatch: i32 [nb][E] counts, [nb][E] first positions, [E] entries
 };
 

@@ -35,7 +35,8 @@ def test_dispatch_tables(cuda, T, E, k):
     inv[perm] = np.arange(len(perm))
     assert np.array_equal(cuda.download(ws + lay.inv, (T * k,), np.int32), inv)
     uniq = np.nonzero(n)[0]
-    assert cuda.download(ws + lay.meta, (2,), np.int32).tolist() == [len(uniq), 0]
+    meta = cuda.download(ws + lay.meta, (3,), np.int32)
+    assert meta[:2].tolist() == [len(uniq), 0]
     assert np.array_equal(cuda.download(ws + lay.uniq, (len(uniq),), np.int32), uniq)
     et = cuda.download(ws + lay.et, (min(T * k, E), 8), np.int32)
     for u, row in enumerate(et):
@@ -44,6 +45,46 @@ def test_dispatch_tables(cuda, T, E, k):
         assert (blob != 0) == (u < len(uniq))
         assert row[2:4].tolist() == ([gs[uniq[u]], n[uniq[u]]] if u < len(uniq) else [0, 0])
         assert row[4:].tolist() == toks + [-1] * (4 - len(toks))
+    # the tile list of the kernels that take the experts in blocks: the GEMM's
+    # of 128 tokens (16 pairs per expert), lp_mid.hip's of 32 (x's images in y)
+    block = 128 if T * k >= 16 * min(E, T * k) else 32 if lay.xf == lay.y else 0
+    if block:
+        tiles = [(u << 16) | b for u, e in enumerate(uniq) for b in range((n[e] + block - 1) // block)]
+        assert meta[2] == len(tiles)
+        assert cuda.download(ws + lay.tiles, (len(tiles),), np.int32).tolist() == tiles
     for p in (ws, dl):
+        cuda.free_device(p)
+    L.free()
+
+
+# experts with exactly a block's tokens, one short of it, one past it, and
+# several blocks: both block sizes, the one-workgroup dispatch and (2049
+# tokens) the three-launch one; 48 tokens: the list of a decode-sized GEMM
+@pytest.mark.parametrize("T,E,counts", [
+    (203, 40, [32, 31, 33, 64, 1]), (2049, 300, [32, 96, 31, 33, 1]), (700, 6, [128, 127, 129, 256, 1]),
+    (2049, 9, [128, 256, 127, 129, 1]), (48, 2, [31]), (48, 3, [16, 32])])
+def test_tile_list_edges(cuda, T, E, counts):
+    L = DeviceLayer(cuda, H=64, I=32, E=E, k=1, group=32, seed=E)
+    logits = np.full((T, E), -5.0, np.float32)
+    logits += 0.1 * np.random.default_rng(T).standard_normal((T, E)).astype(np.float32)
+    at = 0
+    for e, c in enumerate(counts):
+        logits[at:at + c, e] = 5.0
+        logits[at + c:, e] = -50.0
+        at += c
+    lay = lp.ws_layout(L.desc, T)
+    gemm = T >= 16 * E
+    assert gemm or lay.xf == lay.y
+    block = 128 if gemm else 32
+    ws = cuda.alloc_device(lay.total)
+    dl, dx, dh = cuda.upload(logits), cuda.upload(np.ones((T, 64), np.float32)), cuda.alloc_device(T * 64 * 4)
+    L.layer.route_logits(dl, T, ws)
+    L.layer.experts(dx, dh, T, ws)
+    n = np.bincount(logits.argmax(1), minlength=E)
+    assert n[:len(counts)].tolist() == counts
+    want = [(u << 16) | b for u, e in enumerate(np.nonzero(n)[0]) for b in range((n[e] + block - 1) // block)]
+    assert cuda.download(ws + lay.meta, (3,), np.int32).tolist() == [np.count_nonzero(n), 0, len(want)]
+    assert cuda.download(ws + lay.tiles, (len(want),), np.int32).tolist() == want
+    for p in (ws, dl, dx, dh):
         cuda.free_device(p)
     L.free()
