@@ -133,14 +133,15 @@ class Stack:
         return out
 
 
-def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int) -> dict:
+def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int, eager: bool = False) -> dict:
     """Each step decodes a fresh batch of B tokens (resident in HBM): it
     copies the step's B token rows into the stack's residual buffer and
     replays the 48-layer stack captured once as a HIP graph
     (lp_moe_stack_capture).  The same steps are then run eagerly through
     lp_moe_stack_forward (its time is reported too), once more with every
     kernel bracketed by events (per-kernel times), and once with a status
-    readback per layer (the measured unique-expert counts)."""
+    readback per layer (the measured unique-expert counts).  eager: no graph
+    at all, the eager passes stand for it too."""
     import llmpager_amd as lp
     s = stack.s
     ws = cuda.alloc_device(stack.stack.ws_bytes(B))
@@ -150,7 +151,7 @@ def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int) -> dict:
     saved = cuda.upload(h0, s)
     hbuf = cuda.alloc_device(h0.nbytes)
     hcur = cuda.alloc_device(tok_bytes)
-    graph = stack.stack.capture(hcur, B, ws, s)
+    graph = None if eager else stack.stack.capture(hcur, B, ws, s)
 
     def restore():
         cuda.dtod_async(hbuf, saved, h0.nbytes, s)
@@ -158,7 +159,10 @@ def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int) -> dict:
 
     def run_graph(i):
         cuda.dtod_async(hcur, saved + i * tok_bytes, tok_bytes, s)
-        graph.launch(s)
+        if graph is None:
+            stack.step(hcur, B, ws)
+        else:
+            graph.launch(s)
 
     def run(i):
         stack.step(hbuf + i * tok_bytes, B, ws)
@@ -184,7 +188,8 @@ def run_batch(cuda, stack: Stack, B: int, steps: int, warmup: int) -> dict:
     cuda.record_event(e1, s)
     cuda.sync()
     ms_eager = cuda.elapsed_ms(e0, e1)
-    graph.close()
+    if graph is not None:
+        graph.close()
     # the same steps again, each kernel bracketed by events on its stream
     restore()
     cuda.profile_reset()
@@ -953,6 +958,7 @@ def main() -> int:
     ap.add_argument("--shared-only", action="store_true")
     ap.add_argument("--no-step", action="store_true", help="skip the whole decode step leg (attention + MoE)")
     ap.add_argument("--step-only", action="store_true")
+    ap.add_argument("--eager", action="store_true", help="the decode batches without a graph (for counter runs)")
     ap.add_argument("--step-eager", action="store_true", help="time the decode step's eager launches, not a graph")
     ap.add_argument("--paged-layers", type=int, default=P_LAYERS)
     ap.add_argument("--paged-tokens", type=int, default=P_TOKENS)
@@ -1008,7 +1014,7 @@ def main() -> int:
         return 0
     results = {}
     for B in batches:
-        results[B] = run_batch(cuda, stack, B, a.steps, a.warmup)
+        results[B] = run_batch(cuda, stack, B, a.steps, a.warmup, a.eager)
     hl = results[a.headline]
     cpu = None if a.no_cpu else cpu_baseline(stack, a.headline, a.cpu_seconds)
     dom = hl["dominant"]
