@@ -6,8 +6,9 @@
 // expert's weights once (340 MB at H 2048 / I 768 / E 128), so HBM is the
 // floor; what must not happen is a pass over the weights' arithmetic per few
 // tokens.  The decode kernels spend a fifth of the matrix cores' rows on
-// keeping four scales apart and take four tokens per pass (242 + 132 us for
-// gate/up and down of 203 tokens).  Here a token tile is 16 tokens of one
+// keeping four scales apart and take four tokens per pass (235 + 127 us for
+// gate/up and down of 203 tokens, H 2048 / I 768 / 128 experts / top 8; 92 + 53
+// here, traced).  Here a token tile is 16 tokens of one
 // expert and an MFMA's K is exactly one 32-column sub-group:
 //
 //   v_mfma_f32_16x16x32_f16, A = 16 tokens, B = 16 weight rows.  The weights
@@ -26,7 +27,7 @@
 // rows, so a wave holds a whole sub-group of act and gives it its own
 // exponent; down: 64 rows), a workgroup of four waves 128 act columns (256
 // rows of down) for one block of up to 32 tokens of one expert (the tile
-// list of lp_moe_disp_scan: a popular expert's blocks run side by side).
+// list of the dispatch: a popular expert's blocks run side by side).
 //
 // Loads are by whole 128-byte lines: weights in pieces of 256 columns, one
 // piece ahead in registers; a lane's 16 bytes are one sub-group of its row,

@@ -1078,7 +1078,7 @@ static bool bal_down_shape(int I, int group, int entries) {
 // at 4 for H 2048 / I 1408 (500 and 387, 170 and 125 at 4 and 9.4).  Below it
 // lp_mid.hip stays: up to a fifth slower there (188 and 212 at 1, H 4096 / I
 // 1536), but its images carry x to 22 bits where the digits of the one-shot
-// kernels carry 16 (errors 1.3e-6 and 2.6e-5).  The shared MLP of every batch
+// kernels carry 16 (errors 1.5e-6 and 2.5e-5).  The shared MLP of every batch
 // above the decode sizes (all T tokens in one entry) goes there too.
 static bool want_mid(const lp_moe_layer_desc* d, int T) {
     const long pairs = (long)T * d->top_k, maxu = std::min<long>(d->experts, pairs);
