@@ -185,7 +185,7 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
             // x's images end in zero sub-groups, act's rows in the next row:
             // pieces past their last sub-group repeat it, times zero
             const int g = 4 * st + (piece >> 2), gc = MODE == 1 && !SV ? min(g, ng - 1) : g;
-            const uint64_t at = row[t] + 64u * (uint32_t)gc;
+            const uint64_t at = row[t] + 256u * (uint32_t)st - 64u * (uint32_t)(g - gc);
             R.v[t][0] = *gptr<uint4>(at);
             R.v[t][1] = *gptr<uint4>(at + a.lo_off);
             if (MODE == 1) R.e[t] = gc == g ? gptr<int16_t>(a.exps)[(size_t)pos[t] * ng + gc] : 16 * kExpNone;
@@ -212,7 +212,7 @@ __device__ __forceinline__ void mid_tokens(const MidArgs& a, const ExpertEntry& 
     load_scales(0);
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-        row[t] = a.img + (uint64_t)(uint32_t)pos[t] * a.img_stride + 16u * (uint32_t)(piece & 3);
+        row[t] = a.img + (uint64_t)(uint32_t)pos[t] * a.img_stride + 16u * (uint32_t)piece;
         if (MODE == 0) {
             ex[t] = gptr<int>(a.W.xexp)[pos[t]];
         } else {
